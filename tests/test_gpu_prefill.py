@@ -720,3 +720,52 @@ def test_cached_offsets_under_graph_capture(dev):
     with pytest.raises(RuntimeError, match="graph capture"):
         with torch.cuda.graph(g2):
             ops.wkv7_prefill_varlen(pool, ids, fresh, *xs, out=y)
+
+
+@pytest.mark.parametrize("y_dtype", [torch.bfloat16, torch.float32])
+def test_half_and_quarter_heads_bit_identical_to_whole_heads(dev, y_dtype):
+    """Heads split over four workgroups (4 x sequences x heads <= CUs), over
+    two (2 x sequences x heads <= CUs) and not at all: the same sequences
+    beside more and more empty ones give the same bits, which match the
+    oracle. Lengths around the sub-chunk and the pipeline's depth."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    H = 4
+    lens = [1, 15, 16, 17, 111, 0, 112, 113, 400]
+    counts = [cus // (4 * H), cus // (2 * H), cus // (2 * H) + 1]
+    S = max(counts)
+    gen = synthetic.make_generator(97)
+    pool = synthetic.initial_states((S + 1, H, 64, 64), gen)
+    cu = np.concatenate([[0], np.cumsum(lens)]).tolist()
+    vecs = synthetic.wkv7_vectors((cu[-1], H, 64), gen)
+    xs = [vecs[n].to(dev) for n in "rwkvab"]
+    got = []
+    for n in counts:
+        assert n >= len(lens)
+        g = pool.to(dev)
+        y = ops.wkv7_prefill_varlen(g, list(range(1, n + 1)), cu + [cu[-1]] * (n - len(lens)),
+                                    *xs, out_dtype=y_dtype)
+        torch.cuda.synchronize()
+        got.append((y, g))
+    for y, g in got[1:]:
+        assert torch.equal(y, got[0][0]) and torch.equal(g, got[0][1])
+    ids = list(range(1, len(lens) + 1))
+    _check(pool.numpy(), ids, np.array(cu), U.vec_bits(vecs), got[0][1], got[0][0], False)
+
+
+def test_inputs_past_one_gib_of_a_sequence(dev):
+    """A sequence whose inputs pass the 1 GiB at which the row loads move
+    their base forward gives the same bits as its two halves run one after
+    the other (both below it, cut on the 16-token grid)."""
+    H, T, cut = 64, 139_280, 69_664
+    assert T * H * 128 > 1 << 30 > cut * H * 128
+    gen = synthetic.make_generator(11, dev)
+    vecs = synthetic.wkv7_vectors((T, H, 64), gen)
+    xs = [vecs[n] for n in "rwkvab"]
+    h0 = synthetic.initial_states((1, H, 64, 64), gen)
+    h1, ha, hb = (torch.empty_like(h0) for _ in range(3))
+    y = ops.wkv7_prefill_into(h0, h1, [0, T], *xs)
+    ya = ops.wkv7_prefill_into(h0, ha, [0, cut], *[x[:cut] for x in xs])
+    yb = ops.wkv7_prefill_into(ha, hb, [0, T - cut], *[x[cut:] for x in xs])
+    torch.cuda.synchronize()
+    assert torch.isfinite(h1).all()
+    assert torch.equal(y[:cut], ya) and torch.equal(y[cut:], yb) and torch.equal(h1, hb)
