@@ -66,6 +66,14 @@ int wkv7_abi_version(void);
 /* Human-readable text for a return code (WKV7_ERR_* or hipError_t). */
 const char *wkv7_strerror(int code);
 
+/* One layer's vectors of the *_layers entry points (host struct of device
+ * pointers): r, w, k, v, a, b and y as in wkv7_decode_slots /
+ * wkv7_prefill_varlen. */
+struct wkv7_layer_io {
+    const uint16_t *r, *w, *k, *v, *a, *b;
+    void *y;
+};
+
 /*
  * One decode step (one token per slot) for B slots of one layer, in place.
  *
@@ -171,6 +179,25 @@ int wkv7_prefill_varlen(float *wkv_layer, int64_t num_rows, int32_t H,
 #define WKV7_RUN_KV_ZERO 4        /* read k and v as zero */
 #define WKV7_RUN_Y_ALT 8          /* write y to y_alt */
 #define WKV7_RUN_STATE_ALT 16     /* slot_ids[run] is a row of state_alt, not of wkv_layer */
+
+/*
+ * wkv7_decode_slots / wkv7_prefill_varlen for `layers` layers of one bank at
+ * once: layer l's pool starts at wkv + l * layer_stride (floats), its vectors
+ * are io[l] (host array, read before the call returns); the slot ids, offsets
+ * and orders are the same for every layer. Replaces the per-layer loop of
+ * RWKV7Runner.decode_step / prefill around the wkv op
+ * (wkvm/runner/runner.py:41-89). The results are those of the separate calls,
+ * bit for bit; layers must not share state rows.
+ */
+int wkv7_decode_layers(float *wkv, int64_t layer_stride, int32_t layers, int64_t num_rows,
+                       int32_t H, const int32_t *slot_ids, const int32_t *row_order, int32_t B,
+                       const struct wkv7_layer_io *io, int32_t y_dtype, float scale,
+                       void *stream);
+int wkv7_prefill_layers(float *wkv, int64_t layer_stride, int32_t layers, int64_t num_rows,
+                        int32_t H, const int32_t *slot_ids, const int32_t *cu_seqlens,
+                        const int32_t *seq_order, int32_t nseq, int64_t total_tokens,
+                        const struct wkv7_layer_io *io, int32_t y_dtype, int32_t zero_init,
+                        float scale, void *stream);
 
 /*
  * wkv7_prefill_varlen over "runs" with per-run options, for the segmented

@@ -437,3 +437,30 @@ def test_cfg3_fork_then_decode_at_full_size(dev):
     _check_step(before, live, U.vec_bits(vecs), gpool, y)
     assert torch.equal(gpool[dst].cpu(), torch.from_numpy(before[dst]))
     assert not torch.any(gpool[0])
+
+
+@pytest.mark.parametrize("L,B,H", [(1, 1, 1), (3, 5, 2), (33, 4, 3)])
+@pytest.mark.parametrize("y_dtype", [torch.bfloat16, torch.float32])
+def test_all_layers_in_one_launch_equal_one_launch_each(dev, L, B, H, y_dtype):
+    """wkv7_decode_layers gives the bits of wkv7_decode_slots on each layer
+    (33 layers: more than one launch holds), also for vectors that need an
+    aligned copy, and refuses what that refuses."""
+    S = 9
+    gen = synthetic.make_generator(701 + L, dev)
+    wkv = synthetic.initial_states((L, S + 1, H, 64, 64), gen)
+    xs = [synthetic.order(synthetic.wkv7_vectors((B, H, 64), gen)) for _ in range(L)]
+    odd = torch.empty(B * H * 64 + 1, dtype=torch.bfloat16, device=dev)[1:].view(B, H, 64)
+    odd.copy_(xs[-1][0])
+    xs[-1] = (odd, *xs[-1][1:])
+    ids, order = ops.decode_plan(synthetic.active_slots(S, B, synthetic.make_generator(3)), S + 1,
+                                 dev)
+    ref = wkv.clone()
+    ys = ops.wkv7_decode_layers(wkv, ids, xs, out_dtype=y_dtype, row_order=order)
+    for layer in range(L):
+        y = ops.wkv7_decode_slots(ref[layer], ids, *xs[layer], out_dtype=y_dtype, row_order=order)
+        assert torch.equal(ys[layer], y)
+    assert torch.equal(wkv, ref)
+    with pytest.raises(ValueError, match="layers"):
+        ops.wkv7_decode_layers(wkv, ids, xs[1:])
+    with pytest.raises(ValueError, match="bfloat16"):
+        ops.wkv7_decode_layers(wkv, ids, [(x[0].float(), *x[1:]) for x in xs])

@@ -769,3 +769,27 @@ def test_inputs_past_one_gib_of_a_sequence(dev):
     torch.cuda.synchronize()
     assert torch.isfinite(h1).all()
     assert torch.equal(y[:cut], ya) and torch.equal(y[cut:], yb) and torch.equal(h1, hb)
+
+
+@pytest.mark.parametrize("L,H,lens", [(1, 2, [33]), (3, 2, [0, 5, 16]), (33, 1, [17, 1])])
+@pytest.mark.parametrize("y_dtype", [torch.bfloat16, torch.float32])
+def test_all_layers_in_one_launch_equal_one_launch_each(dev, L, H, lens, y_dtype):
+    """wkv7_prefill_layers gives the bits of wkv7_prefill_varlen on each layer
+    (33 layers: more than one launch holds), here on tokens from the fourth
+    on of longer vectors."""
+    n, T, start = len(lens), sum(lens), 3
+    gen = synthetic.make_generator(801 + L, dev)
+    wkv = synthetic.initial_states((L, n + 1, H, 64, 64), gen)
+    xs = [synthetic.order(synthetic.wkv7_vectors((T + 5, H, 64), gen)) for _ in range(L)]
+    ids = torch.arange(1, n + 1, dtype=torch.int32, device=dev)
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device=dev)
+    ref = wkv.clone()
+    ys = [torch.full((T + 5, H, 64), 7.0, dtype=y_dtype, device=dev) for _ in range(L)]
+    ptrs, keep = ops.layer_vectors(xs, (T + 5, H, 64), wkv.device, "prefill")
+    ops.wkv7_prefill_layers(wkv, ids, cu, ptrs, ys, start, T)
+    for layer in range(L):
+        y = ops.wkv7_prefill_varlen(ref[layer], ids, cu, *[x[start:start + T] for x in xs[layer]],
+                                    out_dtype=y_dtype)
+        assert torch.equal(ys[layer][start:start + T], y)
+        assert (ys[layer][:start] == 7).all() and (ys[layer][start + T:] == 7).all()
+    assert torch.equal(wkv, ref)

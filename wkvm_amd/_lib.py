@@ -66,6 +66,10 @@ SIGNATURES = {
     "wkv7_prefill_varlen": (ctypes.c_int, [
         _vp, _i64, _i32, _vp, _vp, _vp, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32,
         _i32, _f32, _vp]),
+    "wkv7_decode_layers": (ctypes.c_int, [
+        _vp, _i64, _i32, _i64, _i32, _vp, _vp, _i32, _vp, _i32, _f32, _vp]),
+    "wkv7_prefill_layers": (ctypes.c_int, [
+        _vp, _i64, _i32, _i64, _i32, _vp, _vp, _vp, _i32, _i64, _vp, _i32, _i32, _f32, _vp]),
     "wkv7_prefill_runs": (ctypes.c_int, [
         _vp, _i64, _i32, _vp, _vp, _vp, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32,
         _i32, _f32, _vp, _vp, _i32, _vp, _i64, _vp, _vp, _i64, _vp, _vp]),

@@ -32,6 +32,10 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
 __device__ __forceinline__ float bf16_lo(uint32_t p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t p) { return __uint_as_float(p & 0xffff0000u); }
 
+// Layers of one *_layers launch (their pointers travel in the kernel
+// arguments: 56 bytes each of 4 KiB).
+constexpr int kMaxLayers = 32;
+
 inline int launch_status() {
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? WKV7_OK : static_cast<int>(e);

@@ -20,6 +20,7 @@
 // (state read from one tensor, written to another; no source = zero state, no
 // destination = the state is not written). A row whose source or destination
 // id is out of range touches no state and gets y = 0.
+#include <algorithm>
 #include <type_traits>
 
 #include "wkv7_common.h"
@@ -98,13 +99,17 @@ __device__ __forceinline__ void store_y(void* y, int64_t io, float yi) {
     static_cast<uint16_t*>(y)[io] = f32_to_bf16(yi);
 }
 
+// One (batch position, head) of a decode launch, a whole workgroup.
 template <bool kF32Out, int kForm>
-__global__ __launch_bounds__(kWave * kDecWaves) void decode_slots_kernel(
-    DecodeIO st, int H, const int32_t* __restrict__ row_order, int B,
-    const uint16_t* __restrict__ r, const uint16_t* __restrict__ w,
-    const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-    const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, void* __restrict__ y,
-    float scale) {
+__device__ __forceinline__ void decode_item(const DecodeIO& st, int H, int64_t pos, int64_t head,
+                                            const int32_t* __restrict__ row_order, int B,
+                                            const uint16_t* __restrict__ r,
+                                            const uint16_t* __restrict__ w,
+                                            const uint16_t* __restrict__ k,
+                                            const uint16_t* __restrict__ v,
+                                            const uint16_t* __restrict__ a,
+                                            const uint16_t* __restrict__ b,
+                                            void* __restrict__ y, float scale) {
   constexpr bool kLoad = kForm == kInPlace || kForm == kSeparate || kForm == kNoOut;
   constexpr bool kStore = kForm == kInPlace || kForm == kSeparate || kForm == kZeroIn;
   __shared__ float4 s_dbkr[kHead];            // (decay, b, k, scale*r) per key row j
@@ -114,8 +119,6 @@ __global__ __launch_bounds__(kWave * kDecWaves) void decode_slots_kernel(
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const int64_t pos = blockIdx.x / H;
-  const int64_t head = blockIdx.x - pos * H;
   int64_t row = pos;
   if (row_order) {
     row = row_order[pos];
@@ -181,6 +184,37 @@ __global__ __launch_bounds__(kWave * kDecWaves) void decode_slots_kernel(
   float* hd = kStore ? st.dst + (dst_slot * H + head) * (kHead * kHead) + wave_off : nullptr;
   const float yi = decode_core<kStore>(hd, h, lane, wave, s_dbkr, s_a, s_p, s_y, vi);
   if (wave == 0) store_y<kF32Out>(y, io, yi);
+}
+
+template <bool kF32Out, int kForm>
+__global__ __launch_bounds__(kWave * kDecWaves) void decode_slots_kernel(
+    DecodeIO st, int H, const int32_t* __restrict__ row_order, int B,
+    const uint16_t* __restrict__ r, const uint16_t* __restrict__ w,
+    const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+    const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, void* __restrict__ y,
+    float scale) {
+  const int64_t pos = blockIdx.x / H;
+  decode_item<kF32Out, kForm>(st, H, pos, blockIdx.x - pos * H, row_order, B, r, w, k, v, a, b, y,
+                              scale);
+}
+
+// Several layers' in-place decode in one launch (grid: B x H, layers). At a
+// few slots a layer's launch is all latency: 12 layers of 4 slots x 12 heads
+// took 12 launches of 4.2 us and as many calls; at 256 slots the launches'
+// ramps and tails between them go (MI355X).
+struct LayerTable {
+  wkv7_layer_io io[kMaxLayers];
+};
+
+template <bool kF32Out>
+__global__ __launch_bounds__(kWave * kDecWaves) void decode_layers_kernel(
+    DecodeIO st, int64_t layer_stride, int H, const int32_t* __restrict__ row_order, int B,
+    float scale, const LayerTable tab) {
+  const int64_t pos = blockIdx.x / H;
+  const wkv7_layer_io& io = tab.io[blockIdx.y];
+  st.src = st.dst = st.dst + blockIdx.y * layer_stride;
+  decode_item<kF32Out, kInPlace>(st, H, pos, blockIdx.x - pos * H, row_order, B, io.r, io.w, io.k,
+                                 io.v, io.a, io.b, io.y, scale);
 }
 
 struct BlockIn {
@@ -340,6 +374,41 @@ extern "C" int wkv7_decode_slots(float* wkv_layer, int64_t num_rows, int32_t H,
   if (B > 0 && (!wkv_layer || !slot_ids)) return WKV7_ERR_ARG;
   const DecodeIO st{wkv_layer, slot_ids, num_rows, wkv_layer, slot_ids, num_rows};
   return launch_decode(st, H, row_order, B, r, w, k, v, a, b, y, y_dtype, scale, stream);
+}
+
+extern "C" int wkv7_decode_layers(float* wkv, int64_t layer_stride, int32_t layers,
+                                  int64_t num_rows, int32_t H, const int32_t* slot_ids,
+                                  const int32_t* row_order, int32_t B, const wkv7_layer_io* io,
+                                  int32_t y_dtype, float scale, void* stream) {
+  if (layers < 0 || B < 0 || H < 1 || num_rows < 1) return WKV7_ERR_ARG;
+  if (y_dtype != WKV7_Y_BF16 && y_dtype != WKV7_Y_F32) return WKV7_ERR_ARG;
+  if (layers == 0 || B == 0) return WKV7_OK;
+  if (!wkv || !slot_ids || !io) return WKV7_ERR_ARG;
+  if (layers > 1 && layer_stride < num_rows * int64_t(H) * kHead * kHead) return WKV7_ERR_SHAPE;
+  for (int32_t l = 0; l < layers; ++l)
+    if (!io[l].r || !io[l].w || !io[l].k || !io[l].v || !io[l].a || !io[l].b || !io[l].y)
+      return WKV7_ERR_ARG;
+  const int64_t row_head = int64_t(B) * H;
+  if (row_head > int64_t(0x7fffffff)) return WKV7_ERR_ARG;
+  hipStream_t s = as_stream(stream);
+  const unsigned threads = kWave * kDecWaves;
+  for (int32_t l = 0; l < layers; l += kMaxLayers) {
+    const int n = std::min(kMaxLayers, layers - l);
+    LayerTable tab{};
+    for (int i = 0; i < n; ++i) tab.io[i] = io[l + i];
+    float* base = wkv + l * layer_stride;
+    const DecodeIO st{base, slot_ids, num_rows, base, slot_ids, num_rows};
+    const dim3 grid(static_cast<unsigned>(row_head), static_cast<unsigned>(n));
+    if (y_dtype == WKV7_Y_F32)
+      decode_layers_kernel<true><<<grid, threads, 0, s>>>(st, layer_stride, H, row_order, B, scale,
+                                                          tab);
+    else
+      decode_layers_kernel<false><<<grid, threads, 0, s>>>(st, layer_stride, H, row_order, B,
+                                                           scale, tab);
+    const int rc = launch_status();
+    if (rc != WKV7_OK) return rc;
+  }
+  return WKV7_OK;
 }
 
 extern "C" int wkv7_decode_into(const float* state_in, int64_t in_rows, const int32_t* in_ids,

@@ -38,11 +38,10 @@ int device_cus() {
   return n;
 }
 
-int prefill_launch(float* wkv_layer, int64_t num_rows, int32_t H, const int32_t* slot_ids,
-                   const int32_t* cu_seqlens, const int32_t* seq_order, int32_t nseq,
-                   int64_t total_tokens, const Inputs& in, void* y, int32_t y_dtype,
-                   int32_t zero_init, float scale, const Runs& runs, void* stream) {
-  const int64_t items = int64_t(nseq) * H, cus = device_cus();
+// p: every field but layers and io, which come from io[0 .. layers).
+int prefill_launch(PrefillArgs& p, int32_t layers, const wkv7_layer_io* io, int32_t y_dtype,
+                   void* stream) {
+  const int64_t items = int64_t(p.nseq) * p.H * layers, cus = device_cus();
   // A launch that leaves half or more of the compute units idle splits each
   // (sequence, head) over two or four workgroups by value columns (same
   // arithmetic per column, so the same bits). A tick is the shorter the fewer
@@ -53,10 +52,10 @@ int prefill_launch(float* wkv_layer, int64_t num_rows, int32_t H, const int32_t*
   const int split = 4 * items <= cus ? 4 : 2 * items <= cus ? 2 : 1;
   const int64_t blocks = items * split;
   if (blocks > int64_t(0x7fffffff)) return WKV7_ERR_ARG;
-  const PrefillArgs p{wkv_layer, num_rows, H, slot_ids, cu_seqlens, seq_order, nseq, in, y,
-                      total_tokens, zero_init, scale, runs};
+  p.layers = layers;
+  for (int32_t l = 0; l < layers; ++l) p.io[l] = io[l];
   hipStream_t s = as_stream(stream);
-  const bool f32 = y_dtype == WKV7_Y_F32, scaled = scale != 1.0f;
+  const bool f32 = y_dtype == WKV7_Y_F32, scaled = p.scale != 1.0f;
   if (split > 1) return prefill_split_launch(split, unsigned(blocks), s, f32, scaled, p);
   return launch_form<WholeHead>(unsigned(blocks), s, f32, scaled, p);
 }
@@ -90,9 +89,40 @@ extern "C" int wkv7_prefill_varlen(float* wkv_layer, int64_t num_rows, int32_t H
   if (total_tokens > 0 && (!r || !w || !k || !v || !a || !b || !y)) return WKV7_ERR_ARG;
   if (!inputs_aligned(r, w, k, v, a, b) || !y_aligned(y, y_dtype)) return WKV7_ERR_SHAPE;
   const Runs runs{nullptr, nullptr, nseq, nullptr, 0, nullptr, nullptr, nullptr, 0};
-  return prefill_launch(wkv_layer, num_rows, H, slot_ids, cu_seqlens, seq_order, nseq,
-                        total_tokens, Inputs{r, w, k, v, a, b}, y, y_dtype, zero_init, scale,
-                        runs, stream);
+  PrefillArgs p{wkv_layer, num_rows,     H,         slot_ids, cu_seqlens, seq_order,
+                nseq,      total_tokens, zero_init, scale,    runs};
+  const wkv7_layer_io io{r, w, k, v, a, b, y};
+  return prefill_launch(p, 1, &io, y_dtype, stream);
+}
+
+extern "C" int wkv7_prefill_layers(float* wkv, int64_t layer_stride, int32_t layers,
+                                   int64_t num_rows, int32_t H, const int32_t* slot_ids,
+                                   const int32_t* cu_seqlens, const int32_t* seq_order,
+                                   int32_t nseq, int64_t total_tokens, const wkv7_layer_io* io,
+                                   int32_t y_dtype, int32_t zero_init, float scale,
+                                   void* stream) {
+  if (layers < 0 || nseq < 0 || H < 1 || num_rows < 1 || total_tokens < 0) return WKV7_ERR_ARG;
+  if (y_dtype != WKV7_Y_BF16 && y_dtype != WKV7_Y_F32) return WKV7_ERR_ARG;
+  if (layers == 0 || nseq == 0) return WKV7_OK;
+  if (!wkv || !slot_ids || !cu_seqlens || !io) return WKV7_ERR_ARG;
+  if (layers > 1 && layer_stride < num_rows * int64_t(H) * kHead * kHead) return WKV7_ERR_SHAPE;
+  for (int32_t l = 0; l < layers; ++l) {
+    const wkv7_layer_io& x = io[l];
+    if (total_tokens > 0 && (!x.r || !x.w || !x.k || !x.v || !x.a || !x.b || !x.y))
+      return WKV7_ERR_ARG;
+    if (!inputs_aligned(x.r, x.w, x.k, x.v, x.a, x.b) || !y_aligned(x.y, y_dtype))
+      return WKV7_ERR_SHAPE;
+  }
+  const Runs runs{nullptr, nullptr, nseq, nullptr, 0, nullptr, nullptr, nullptr, 0};
+  for (int32_t l = 0; l < layers; l += kMaxLayers) {
+    const int32_t n = layers - l < kMaxLayers ? layers - l : kMaxLayers;
+    PrefillArgs p{wkv + l * layer_stride, num_rows,     H,         slot_ids, cu_seqlens, seq_order,
+                  nseq,                   total_tokens, zero_init, scale,    runs};
+    p.layer_stride = layer_stride;
+    const int rc = prefill_launch(p, n, io + l, y_dtype, stream);
+    if (rc != WKV7_OK) return rc;
+  }
+  return WKV7_OK;
 }
 
 extern "C" int wkv7_prefill_runs(float* wkv_layer, int64_t num_rows, int32_t H,
@@ -120,9 +150,10 @@ extern "C" int wkv7_prefill_runs(float* wkv_layer, int64_t num_rows, int32_t H,
     return WKV7_ERR_SHAPE;
   const Runs runs{run_flags, cu_alt,   n_primary, state_alt, alt_rows,
                   y_alt ? y_alt : y, state_in, in_ids,    in_rows};
-  return prefill_launch(wkv_layer, num_rows, H, slot_ids, cu_seqlens, seq_order, nseq,
-                        total_tokens, Inputs{r, w, k, v, a, b}, y, y_dtype, zero_init, scale,
-                        runs, stream);
+  PrefillArgs p{wkv_layer, num_rows,     H,         slot_ids, cu_seqlens, seq_order,
+                nseq,      total_tokens, zero_init, scale,    runs};
+  const wkv7_layer_io io{r, w, k, v, a, b, y};
+  return prefill_launch(p, 1, &io, y_dtype, stream);
 }
 
 extern "C" int wkv7_prefill_into(const float* state_in, int64_t in_rows, const int32_t* in_ids,
@@ -143,7 +174,8 @@ extern "C" int wkv7_prefill_into(const float* state_in, int64_t in_rows, const i
   if (!inputs_aligned(r, w, k, v, a, b) || !y_aligned(y, y_dtype)) return WKV7_ERR_SHAPE;
   // no state_in: zero initial state; no state_out: no final state written
   const Runs runs{nullptr, nullptr, nseq, nullptr, 0, nullptr, state_in, in_ids, in_rows};
-  return prefill_launch(state_out, state_out ? out_rows : 0, H, out_ids, cu_seqlens, seq_order,
-                        nseq, total_tokens, Inputs{r, w, k, v, a, b}, y, y_dtype,
-                        state_in ? 0 : 1, scale, runs, stream);
+  PrefillArgs p{state_out, state_out ? out_rows : 0, H,                out_ids, cu_seqlens, seq_order,
+                nseq,      total_tokens,             state_in ? 0 : 1, scale,   runs};
+  const wkv7_layer_io io{r, w, k, v, a, b, y};
+  return prefill_launch(p, 1, &io, y_dtype, stream);
 }

@@ -238,18 +238,22 @@ struct Runs {
   int64_t in_rows;
 };
 
+// `layers` layers share the plan: layer l's states are at wkv + l *
+// layer_stride, its vectors io[l] (one launch instead of a layer's launch
+// after the other's tail).
 struct PrefillArgs {
   float* wkv;  // final states, and initial ones unless runs.state_in or zero_init; null: none
   int64_t num_rows;
   int H;
   const int32_t *slot_ids, *cu_seqlens, *seq_order;  // slot_ids null: run s is row s
   int nseq;
-  Inputs in;
-  void* y;
   int64_t total_tokens;
   int zero_init;
   float scale;
   Runs runs;
+  int layers;
+  int64_t layer_stride;
+  wkv7_layer_io io[kMaxLayers];
 };
 
 // Launches the forms of wkv7_prefill_split.hip: `split` (2 or 4) workgroups
@@ -898,8 +902,12 @@ __global__ __launch_bounds__(kWaves * kWave) void prefill_kernel(const PrefillAr
   // so the role branches are scalar branches
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   const int64_t item = blockIdx.x / kSplit;
-  const int64_t pos = item / p.H;
-  const int64_t head = item - pos * p.H;
+  // sequences outermost: the longest ones of every layer start first
+  const int64_t per_seq = int64_t(p.layers) * p.H;
+  const int64_t pos = item / per_seq;
+  const int64_t layer = (item - pos * per_seq) / p.H;
+  const int64_t head = item - pos * per_seq - layer * p.H;
+  const wkv7_layer_io& io = p.io[layer];
   const int64_t seq = p.seq_order ? int64_t(p.seq_order[pos]) : pos;
   if (seq < 0 || seq >= p.nseq) return;  // uniform: the whole block leaves
   const Runs& runs = p.runs;
@@ -916,11 +924,11 @@ __global__ __launch_bounds__(kWaves * kWave) void prefill_kernel(const PrefillAr
   g.tstride = int64_t(p.H) * kHead;
   g.hoff = head * kHead;
   const int64_t n_sub = (g.t_end - g.t_beg + kSub - 1) / kSub;
-  void* yb = (fl & WKV7_RUN_Y_ALT) ? runs.y_alt : p.y;
+  void* yb = (fl & WKV7_RUN_Y_ALT) ? runs.y_alt : io.y;
 
   // State rows of this run: checked before any state access (uniform).
   const bool state_alt = fl & WKV7_RUN_STATE_ALT;
-  float* out_base = state_alt ? runs.state_alt : p.wkv;
+  float* out_base = state_alt ? runs.state_alt : p.wkv ? p.wkv + layer * p.layer_stride : nullptr;
   const int64_t out_rows = state_alt ? runs.alt_rows : p.num_rows;
   const int64_t slot = p.slot_ids ? int64_t(p.slot_ids[seq]) : seq;
   const bool from_eye = fl & WKV7_RUN_INIT_IDENTITY;
@@ -954,7 +962,7 @@ __global__ __launch_bounds__(kWaves * kWave) void prefill_kernel(const PrefillAr
     else if (role == kInverse)
       inverse_role(sm, n_sub, lane);
     else if (role == kIo)
-      io_role(sm, p.in, g, n_sub, lane, fl & WKV7_RUN_KV_ZERO);
+      io_role(sm, Inputs{io.r, io.w, io.k, io.v, io.a, io.b}, g, n_sub, lane, fl & WKV7_RUN_KV_ZERO);
     else
       for (int64_t k = 0; k < n_sub + 5; ++k) end_tick();  // no work: every tick's barrier
   }

@@ -38,6 +38,7 @@ class DecodeGraph:
         self.bank, self.batch_size = bank, batch_size
         # slot ids in [0, B), visiting order in [B, 2B); the pad row 0 until set
         self.plan = torch.zeros(2 * batch_size, dtype=torch.int32, device=dev)
+        self._slots_set = torch.cuda.Event()
         self.plan[batch_size:] = torch.arange(batch_size, dtype=torch.int32, device=dev)
         # inputs[l] = (r, w, k, v, a, b), each [B, H, 64] bf16 (w = log-decay)
         self.inputs = torch.zeros((L, 6, batch_size, H, HEAD_SIZE), dtype=torch.bfloat16,
@@ -72,10 +73,11 @@ class DecodeGraph:
                              f"{self.batch_size}")
         lst = ops.host_ids(ids, self.bank.num_slots + 1, "slot_ids", distinct=True)
         order = sorted(range(len(lst)), key=lst.__getitem__)
-        self.plan.copy_(torch.tensor(lst + order, dtype=torch.int32))
+        ops.refresh_ints(self.plan, lst + order, self._slots_set)
 
     def replay(self) -> torch.Tensor:
         """Run the captured step; returns the static ``y`` [L, B, H, 64]."""
+        torch.cuda.current_stream(self.bank.device).wait_event(self._slots_set)
         self.graph.replay()
         return self.y
 

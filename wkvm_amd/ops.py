@@ -23,6 +23,7 @@ Error behaviour mirrors the reference: invalid arguments raise ``ValueError``
 
 from __future__ import annotations
 
+import ctypes
 import threading
 from collections import OrderedDict
 from typing import Iterable, Sequence
@@ -83,8 +84,31 @@ def host_ids(ids, rows: int, what: str, distinct: bool) -> list[int]:
     return out
 
 
-def device_ids(ids, rows: int, device: torch.device, what: str, distinct: bool = True) -> torch.Tensor:
-    """Slot ids as a device int32 tensor.
+def upload_ints(values: list[int], device: torch.device, wait: bool = True) -> torch.Tensor:
+    """Host integers as a device int32 tensor. With ``wait`` it is complete on
+    return and any stream may use it. Without, it is only ordered on the
+    current stream: the copy runs from pinned memory (kept by torch until it
+    is done) and the host does not wait for the stream's earlier work, as a
+    copy from pageable memory makes it do (a fork's four id uploads: 80 us of
+    its 240). For ids that a call uses itself and does not hand out. Under graph
+    capture the waiting form is used, which capture refuses: a replay would
+    read pinned memory that may hold other values by then."""
+    if wait or torch.cuda.is_current_stream_capturing():
+        return torch.tensor(values, dtype=torch.int32, device=device)
+    return torch.tensor(values, dtype=torch.int32, pin_memory=True).to(device, non_blocking=True)
+
+
+def refresh_ints(dst: torch.Tensor, values: list[int], event: torch.cuda.Event) -> None:
+    """Host integers into a device int32 tensor that a graph reads, ordered on
+    the current stream without waiting for it; ``event`` is recorded behind
+    the copy, for a replay on another stream to wait for."""
+    dst.copy_(torch.tensor(values, dtype=torch.int32, pin_memory=True), non_blocking=True)
+    event.record(torch.cuda.current_stream(dst.device))
+
+
+def device_ids(ids, rows: int, device: torch.device, what: str, distinct: bool = True,
+               wait: bool = True) -> torch.Tensor:
+    """Slot ids as a device int32 tensor (``wait`` as in ``upload_ints``).
 
     Host ids (list / tuple / numpy / CPU tensor) are validated first and raise
     ``ValueError``. A CUDA int32 tensor is taken as already validated: the
@@ -97,12 +121,13 @@ def device_ids(ids, rows: int, device: torch.device, what: str, distinct: bool =
         if ids.device != device:
             raise ValueError(f"{what}: ids on {ids.device}, pool on {device}")
         return ids
-    lst = host_ids(ids, rows, what, distinct)
-    return torch.tensor(lst, dtype=torch.int32, device=device)
+    return upload_ints(host_ids(ids, rows, what, distinct), device, wait)
 
 
-def decode_plan(slot_ids, rows: int, device: torch.device) -> tuple[torch.Tensor, torch.Tensor | None]:
-    """Device ``(slot_ids, row_order)`` for a decode batch.
+def decode_plan(slot_ids, rows: int, device: torch.device, wait: bool = True,
+                ) -> tuple[torch.Tensor, torch.Tensor | None]:
+    """Device ``(slot_ids, row_order)`` for a decode batch (``wait`` as in
+    ``upload_ints``).
 
     Host ids are validated (in range, distinct) and uploaded together with the
     batch rows sorted by slot id -- the visiting order that keeps the kernel's
@@ -112,7 +137,7 @@ def decode_plan(slot_ids, rows: int, device: torch.device) -> tuple[torch.Tensor
         return device_ids(slot_ids, rows, device, "slot_ids"), None
     lst = host_ids(slot_ids, rows, "slot_ids", distinct=True)
     order = sorted(range(len(lst)), key=lst.__getitem__)
-    both = torch.tensor(lst + order, dtype=torch.int32, device=device)
+    both = upload_ints(lst + order, device, wait)
     return both[:len(lst)], both[len(lst):]
 
 
@@ -167,7 +192,7 @@ def wkv7_decode_slots(wkv_layer: torch.Tensor, slot_ids, r, w, k, v, a, b, *,
     """
     rows, H = _check_pool(wkv_layer)
     dev = wkv_layer.device
-    ids, order = decode_plan(slot_ids, rows, dev)
+    ids, order = decode_plan(slot_ids, rows, dev, wait=False)
     if row_order is not None:
         if not (isinstance(row_order, torch.Tensor) and row_order.is_cuda
                 and row_order.dtype == torch.int32 and row_order.shape == ids.shape):
@@ -235,9 +260,10 @@ def wkv7_decode_into(state_in: torch.Tensor | None, state_out: torch.Tensor | No
         dst = list(range(B)) if out_ids is None else [int(i) for i in out_ids]
         if src != dst and set(src) & set(dst):
             raise ValueError("a row writes a state row that another row reads")
-    d_in = None if in_ids is None else device_ids(in_ids, in_rows, dev, "in_ids", distinct=False)
+    d_in = None if in_ids is None else device_ids(in_ids, in_rows, dev, "in_ids", distinct=False,
+                                                  wait=False)
     d_out = None if out_ids is None else device_ids(out_ids, out_rows, dev, "out_ids",
-                                                    distinct=True)
+                                                    distinct=True, wait=False)
     for ids in (d_in, d_out):
         if ids is not None and int(ids.shape[0]) != B:
             raise ValueError(f"{int(ids.shape[0])} ids for {B} batch rows")
@@ -341,7 +367,7 @@ def wkv7_prefill_varlen(wkv_layer: torch.Tensor, slot_ids, cu_seqlens, r, w, k, 
     """
     rows, H = _check_pool(wkv_layer)
     dev = wkv_layer.device
-    ids = device_ids(slot_ids, rows, dev, "slot_ids", distinct=True)
+    ids = device_ids(slot_ids, rows, dev, "slot_ids", distinct=True, wait=False)
     nseq = int(ids.shape[0])
     _require_cuda(r, "prefill.r")
     T = int(r.shape[0]) if r.dim() == 3 else -1
@@ -375,6 +401,118 @@ def wkv7_prefill_varlen(wkv_layer: torch.Tensor, slot_ids, cu_seqlens, r, w, k, 
                                          int(bool(zero_init)), float(scale), _stream_ptr(dev))
     _lib.check(rc, "wkv7_prefill_varlen")
     return y
+
+
+# -- every layer of a bank in one launch -------------------------------------------
+
+def check_bank(wkv: torch.Tensor) -> tuple[int, int, int, int]:
+    """``(layers, rows, H, layer stride in elements)`` of a bank's ``[L, rows,
+    H, 64, 64]`` state tensor."""
+    _require_cuda(wkv, "wkv")
+    if wkv.dim() != 5:
+        raise ValueError(f"wkv must be [layers, rows, H, 64, 64], got {tuple(wkv.shape)}")
+    rows, H = _check_pool(wkv[0])
+    if wkv.shape[0] > 1 and wkv.stride(0) < wkv[0].numel():
+        raise ValueError("the bank's layers overlap")
+    return int(wkv.shape[0]), rows, H, int(wkv.stride(0))
+
+
+def layer_vectors(layer_inputs, shape: tuple[int, ...], device: torch.device, what: str,
+                  ) -> tuple[list[list[int]], list]:
+    """Device pointers ``[[r, w, k, v, a, b], ...]`` of each layer's vectors and
+    the tensors they belong to (contiguous 16-byte aligned copies where a
+    vector needs one)."""
+    ptrs, keep = [], []
+    for xs in layer_inputs:
+        if len(xs) != 6:
+            raise ValueError(f"{what}: a layer's inputs are (r, w, k, v, a, b), got {len(xs)}")
+        row = []
+        for x in xs:
+            if not (isinstance(x, torch.Tensor) and x.dtype is torch.bfloat16
+                    and x.shape == shape and x.device == device and x.is_contiguous()):
+                break
+            p = x.data_ptr()
+            if p & 15:
+                break
+            row.append(p)
+        else:
+            ptrs.append(row)
+            continue
+        xs = _check_vectors(xs, shape, device, what)  # names the fault, or copies
+        keep.append(xs)
+        ptrs.append([x.data_ptr() for x in xs])
+    return ptrs, keep
+
+
+def _io_table(ptrs: list[list[int]], ys: Sequence[int], offset: int = 0):
+    """``struct wkv7_layer_io`` array, the vectors ``offset`` bytes in."""
+    flat = []
+    for row, y in zip(ptrs, ys):
+        flat += [p + offset for p in row] if offset else row
+        flat.append(y)
+    return (ctypes.c_void_p * len(flat))(*flat)
+
+
+def wkv7_decode_layers(wkv: torch.Tensor, ids: torch.Tensor, layer_inputs, *,
+                       scale: float = 1.0, out_dtype: torch.dtype = torch.bfloat16,
+                       row_order: torch.Tensor | None = None) -> list[torch.Tensor]:
+    """``wkv7_decode_slots`` of every layer of ``wkv [L, rows, H, 64, 64]`` in
+    one launch: ``layer_inputs[l]`` are layer l's ``(r, w, k, v, a, b)``
+    ``[B, H, 64]``; ``ids`` and ``row_order`` are device int32 (see
+    ``decode_plan``). Returns the layers' ``y [B, H, 64]``, views of one
+    ``[L, B, H, 64]`` tensor."""
+    L, rows, H, stride = check_bank(wkv)
+    dev = wkv.device
+    if len(layer_inputs) != L:
+        raise ValueError(f"expected inputs for {L} layers, got {len(layer_inputs)}")
+    ids = device_ids(ids, rows, dev, "slot_ids")
+    B = int(ids.shape[0])
+    if row_order is not None and not (isinstance(row_order, torch.Tensor) and row_order.is_cuda
+                                      and row_order.dtype == torch.int32
+                                      and row_order.shape == ids.shape):
+        raise ValueError("row_order must be a device int32 tensor shaped like slot_ids")
+    ptrs, keep = layer_vectors(layer_inputs, (B, H, HEAD_SIZE), dev, "decode")
+    code = _y_code(out_dtype)
+    y = torch.empty((L, B, H, HEAD_SIZE), dtype=out_dtype, device=dev)
+    if B:
+        base, step = y.data_ptr(), B * H * HEAD_SIZE * y.element_size()
+        io = _io_table(ptrs, [base + l * step for l in range(L)])
+        rc = _lib.load().wkv7_decode_layers(wkv.data_ptr(), stride, L, rows, H, ids.data_ptr(),
+                                            _ptr(row_order), B, io, code, float(scale),
+                                            _stream_ptr(dev))
+        _lib.check(rc, "wkv7_decode_layers")
+    return list(y.unbind(0))
+
+
+def wkv7_prefill_layers(wkv: torch.Tensor, ids: torch.Tensor, cu_seqlens: torch.Tensor,
+                        ptrs: list[list[int]], ys: Sequence[torch.Tensor], start: int, n: int, *,
+                        zero_init: bool = False, scale: float = 1.0,
+                        seq_order: torch.Tensor | None = None) -> None:
+    """``wkv7_prefill_varlen`` of every layer of ``wkv [L, rows, H, 64, 64]`` in
+    one launch, on tokens ``[start, start + n)`` of the layers' vectors
+    (``ptrs`` from ``layer_vectors``) and outputs ``ys [T, H, 64]``.
+    ``cu_seqlens`` (device int32, relative to ``start``), ``ids`` and
+    ``seq_order`` are the same for every layer."""
+    L, rows, H, stride = check_bank(wkv)
+    dev = wkv.device
+    if len(ptrs) != L or len(ys) != L:
+        raise ValueError(f"expected inputs for {L} layers, got {len(ptrs)}")
+    ids = device_ids(ids, rows, dev, "slot_ids")
+    nseq = int(ids.shape[0])
+    for t, what, size in ((cu_seqlens, "cu_seqlens", nseq + 1), (seq_order, "seq_order", nseq)):
+        if t is not None and not (t.is_cuda and t.dtype == torch.int32
+                                  and tuple(t.shape) == (size,)):
+            raise ValueError(f"{what} must be a device int32 tensor of {size} entries")
+    if nseq == 0:
+        return
+    token = H * HEAD_SIZE
+    out = start * token * ys[0].element_size()
+    io = _io_table(ptrs, [y.data_ptr() + out for y in ys], start * token * 2)
+    rc = _lib.load().wkv7_prefill_layers(wkv.data_ptr(), stride, L, rows, H, ids.data_ptr(),
+                                         cu_seqlens.data_ptr(), _ptr(seq_order), nseq, n, io,
+                                         _y_code(ys[0].dtype), int(bool(zero_init)), float(scale),
+                                         _stream_ptr(dev))
+    _lib.check(rc, "wkv7_prefill_layers")
 
 
 def wkv7_prefill_into(state_in: torch.Tensor | None, state_out: torch.Tensor | None,
@@ -416,9 +554,10 @@ def wkv7_prefill_into(state_in: torch.Tensor | None, state_out: torch.Tensor | N
         dst = list(range(nseq)) if out_ids is None else [int(i) for i in out_ids]
         if src != dst and set(src) & set(dst):
             raise ValueError("a sequence writes a state row that another sequence reads")
-    d_in = None if in_ids is None else device_ids(in_ids, in_rows, dev, "in_ids", distinct=False)
+    d_in = None if in_ids is None else device_ids(in_ids, in_rows, dev, "in_ids", distinct=False,
+                                                  wait=False)
     d_out = None if out_ids is None else device_ids(out_ids, out_rows, dev, "out_ids",
-                                                    distinct=True)
+                                                    distinct=True, wait=False)
     for ids in (d_in, d_out):
         if ids is not None and int(ids.shape[0]) != nseq:
             raise ValueError(f"{int(ids.shape[0])} ids for {nseq} sequences")
@@ -552,7 +691,7 @@ def wkv7_prefill_segments(wkv_layer: torch.Tensor, slot_ids, cu_seqlens, r, w, k
     order = sorted(range(nruns), key=lambda i: -lens[i])
     parts = [run_slot + alt_slot, run_flags + alt_flags, prim_cu, alt_pairs or [0, 0], order,
              seq_tab or [0, 0, 0], seg_tab or [0, 0], blk, run_src + [0] * len(alt_slot)]
-    plan = torch.tensor([x for p in parts for x in p], dtype=torch.int32, device=dev)
+    plan = upload_ints([x for p in parts for x in p], dev, wait=False)
     views, at = [], 0
     for p in parts:
         views.append(plan[at:at + len(p)])
@@ -647,8 +786,9 @@ def slot_copy(dst: torch.Tensor, dst_ids, src: torch.Tensor, src_ids, slot_dim: 
     if isinstance(dst_ids, list) and isinstance(src_ids, list) and _overlaps(dst, src):
         if set(dst_ids) & set(src_ids):
             raise ValueError("fork destination rows overlap source rows")
-    d_t = device_ids(dst_ids, d_rows, dev, "dst_ids") if dst_ids is not None else None
-    s_t = device_ids(src_ids, s_rows, dev, "src_ids", distinct=False) if src_ids is not None else None
+    d_t = device_ids(dst_ids, d_rows, dev, "dst_ids", wait=False) if dst_ids is not None else None
+    s_t = (device_ids(src_ids, s_rows, dev, "src_ids", distinct=False, wait=False)
+           if src_ids is not None else None)
     if n is None:
         n = int((d_t if d_t is not None else s_t).shape[0])
     if d_t is None and n > d_rows:
@@ -742,7 +882,7 @@ def slot_zero(t: torch.Tensor, ids, slot_dim: int) -> None:
     """Zero slot rows ``ids`` of ``t`` along ``slot_dim`` with a fill kernel."""
     _require_cuda(t, "tensor")
     outer, os_, ss, rows, rb = slot_view(t, slot_dim)
-    ids_t = device_ids(ids, rows, t.device, "ids", distinct=False)
+    ids_t = device_ids(ids, rows, t.device, "ids", distinct=False, wait=False)
     n = int(ids_t.shape[0])
     if n == 0:
         return
@@ -1053,6 +1193,18 @@ def _fla_state(initial_state, nseq: int, H: int, dev: torch.device) -> torch.Ten
     return initial_state.to(device=dev, dtype=torch.float32).contiguous()
 
 
+def _vector_ptrs(xs, shape, device: torch.device) -> list[int] | None:
+    """Device pointers of vectors the kernels can read as they are (bf16,
+    contiguous, 16-byte aligned, all of ``shape``), else None."""
+    ptrs = []
+    for x in xs:
+        if not (isinstance(x, torch.Tensor) and x.dtype is torch.bfloat16 and x.shape == shape
+                and x.device == device and x.is_contiguous()):
+            return None
+        ptrs.append(x.data_ptr())
+    return None if any(p & 15 for p in ptrs) else ptrs
+
+
 def _seq_op(r, w, k, v, a, b, scale, initial_state, output_final_state, cu_seqlens, head_first):
     """fla's wkv-op contract: ``[B, T, H, 64]`` inputs (or ``[1, T_total, H,
     64]`` packed by ``cu_seqlens``), ``initial_state`` read, a new
@@ -1069,21 +1221,43 @@ def _seq_op(r, w, k, v, a, b, scale, initial_state, output_final_state, cu_seqle
         raise ValueError(f"head size must be {HEAD_SIZE}, got {K}")
     if r.dtype != torch.bfloat16:
         raise ValueError("the gfx950 WKV7 kernels take bfloat16 inputs")
+    dev = r.device
+    ptrs = None if head_first else _vector_ptrs((r, w, k, v, a, b), r.shape, dev)
     if cu_seqlens is None:
         nseq = B
         host_cu = [i * T for i in range(B + 1)]
-        flat = [x.reshape(B * T, H, K) for x in (r, w, k, v, a, b)]
     else:
         if B != 1:
             raise ValueError("cu_seqlens requires batch size 1 (packed sequences)")
         # fla passes a device LongTensor; the offsets are validated on the host
         host_cu = _host_cu(cu_seqlens, T)
         nseq = len(host_cu) - 1
-        flat = [x[0] for x in (r, w, k, v, a, b)]
-    dev = r.device
     state = _fla_state(initial_state, nseq, H, dev)
     lens = [host_cu[i + 1] - host_cu[i] for i in range(nseq)]
-    if nseq and all(n == 1 for n in lens):  # decode: one token per sequence
+    decode = nseq > 0 and max(lens) == 1 == min(lens)  # one token per sequence
+    if ptrs and nseq and (decode or auto_segments(H, lens, dev) == 1) and r.dtype == torch.bfloat16:
+        # every argument is checked: straight to the launch
+        lib = _lib.load()
+        final = (torch.empty((nseq, H, K, K), dtype=torch.float32, device=dev)
+                 if output_final_state else None)
+        y = torch.empty((B, T, H, K), dtype=torch.bfloat16, device=dev)
+        states = (_ptr(state), 0 if state is None else nseq, None,
+                  _ptr(final), 0 if final is None else nseq, None, H)
+        tail = (y.data_ptr(), _lib.WKV7_Y_BF16, float(scale), _stream_ptr(dev))
+        if decode:
+            rc = lib.wkv7_decode_into(*states, None, nseq, *ptrs, *tail)
+            _lib.check(rc, "wkv7_decode_into")
+        else:
+            plan = _device_plan(host_cu, dev).data_ptr()
+            rc = lib.wkv7_prefill_into(*states, plan, plan + 4 * (nseq + 1), nseq, host_cu[-1],
+                                       *ptrs, *tail)
+            _lib.check(rc, "wkv7_prefill_into")
+        return y, final
+    if cu_seqlens is None:
+        flat = [x.reshape(B * T, H, K) for x in (r, w, k, v, a, b)]
+    else:
+        flat = [x[0] for x in (r, w, k, v, a, b)]
+    if decode:
         final = (torch.empty((nseq, H, K, K), dtype=torch.float32, device=dev)
                  if output_final_state else None)
         y = wkv7_decode_into(state, final, *flat, scale=scale, out_dtype=r.dtype)

@@ -270,6 +270,7 @@ class TimeMixDecodeGraph:
         # [2B, 3B] offsets 0..B
         self.plan = torch.cat([torch.arange(1, B + 1), torch.arange(B),
                                torch.arange(B + 1)]).to(torch.int32).to(dev)
+        self._slots_set = torch.cuda.Event()
         self.x = torch.zeros((len(layers), B, D), dtype=torch.bfloat16, device=dev)
         self.o: list[torch.Tensor] = []
         batch = TokenBatch(self.plan[:B], self.plan[2 * B:], self.plan[B:2 * B], B, B, True)
@@ -306,9 +307,10 @@ class TimeMixDecodeGraph:
             raise ValueError(f"batch of {len(lst)} slots for a graph of batch size "
                              f"{self.batch_size}")
         order = sorted(range(len(lst)), key=lst.__getitem__)
-        self.plan[:2 * self.batch_size].copy_(torch.tensor(lst + order, dtype=torch.int32))
+        ops.refresh_ints(self.plan[:2 * self.batch_size], lst + order, self._slots_set)
 
     def replay(self) -> list[torch.Tensor]:
         """Run the captured step; returns the static outputs ``o`` (L x [B, D])."""
+        torch.cuda.current_stream(self.bank.device).wait_event(self._slots_set)
         self.graph.replay()
         return self.o
