@@ -182,3 +182,18 @@ def test_split_k_over_several_groups(dev):
     y1, y2 = ops.proj_grouped([(x1, w1), (x2, w2, b2, "sigmoid")], outs=ys)
     _assert_within_one_ulp(y1, _exact(x1, w1, None, None))
     _assert_within_one_ulp(y2, _exact(x2, w2, b2, "sigmoid"))
+
+
+@pytest.mark.parametrize("M", [31, 65, 127, 129, 385, 511])
+def test_every_tile_shape_of_long_k(dev, M):
+    """Row counts that take each tile shape of long products (32 x 32, 64 x 32,
+    128 x 64, the last over one and two rounds), with partial tiles in both
+    directions and a k tail."""
+    gen = torch.Generator().manual_seed(53)
+    K = 1056
+    prods = []
+    for n, act in ((2040, None), (2048, None), (1000, "tanh"), (100, "sigmoid")):
+        prods.append((_rand((M, K), gen, dev), _rand((n, K), gen, dev, 1 / math.sqrt(K)),
+                      _rand((n,), gen, dev), act))
+    for y, (x, w, b, act) in zip(ops.proj_grouped(prods), prods):
+        _assert_within_one_ulp(y, _exact(x, w, b, act))

@@ -8,7 +8,7 @@
 // the workgroups of all groups form one grid, each computing a BM x BN output
 // tile over the whole k.
 //
-// Workgroup: GM x GN waves (4 or 8), each a (BM/GM) x (BN/GN) block of
+// Workgroup: GM x GN waves (4, 8 or 16), each a (BM/GM) x (BN/GN) block of
 // 16 x 16 accumulator tiles on v_mfma_f32_16x16x32_bf16. Operand layout of
 // that instruction (lane l, li = l % 16, lg = l / 16): A lane holds
 // A[li][8lg .. 8lg+7] of a 32-wide k block, B lane holds B[8lg .. 8lg+7][li],
@@ -406,34 +406,42 @@ Plan make_plan(int64_t m, const wkv7_proj_group* gs, int ng, int cus) {
     cols += gs[i].n;
   }
   // The launch reads (BM + BN) rows of k per tile from L2, which bounds it
-  // at a few hundred rows. With long k (8 stages or more), the largest tile
-  // of one workgroup per compute unit that fills three quarters of the units
-  // or more in one round: 128 x 64 (8 waves, 3-stage ring of 128-wide k
-  // stages, 144 KiB of LDS), then 64 x 32 (4 waves, 4-stage ring, 96 KiB).
-  // A unit then reads 192 or 96 rows instead of twice 128 or 64 (the 1.5B
-  // first stage at 256 rows: 20.1 against 22.7 us; o_proj 10.6 against 11.3).
-  // Else 64 x 64 tiles (8 waves, 2-stage ring) when they give every unit
-  // about 1.5 workgroups or more; else 32 x 32 tiles (4 waves, 4-stage ring).
+  // at a few hundred rows. With long k, the shape whose rounds over the
+  // compute units take least; us per round, measured at k = 2048 (128 x 64: 16
+  // waves, 3-stage ring of 128-wide k stages, 144 KiB of LDS, one workgroup per
+  // unit; 64 x 32: 8 waves, 4-stage ring, 96 KiB, one; 32 x 32: 4 waves,
+  // 4-stage ring, 64 KiB, two). The 1.5B first stage: 8 rows 8.1 us in 32 x 32
+  // tiles (9.3 in 64 x 32 with 4 waves), 64 rows 9.3 in 64 x 32 (10.3), 256 rows
+  // 18.6 in 128 x 64 (19.6 with 8 waves), 512 rows 33.9 (39.5 in 64 x 64);
+  // o_proj at 256 rows 9.1 (9.8 with 4 waves), at 512 rows 14.1 (17.0 in 32 x 32).
+  // With short k the prologue counts as much as the stages: 64 x 64 tiles (8
+  // waves, 2-stage ring) as soon as every unit gets one (LoRA up-projections at
+  // 128 rows 5.2 against 7.1 us), else 32 x 32.
   Plan p{1, 1, 0};
   int64_t tiles = count_tiles(m, gs, ng, kShapes[1]);
-  auto fills = [&](int64_t t) { return t * 4 >= int64_t(cus) * 3 && t <= int64_t(cus); };
-  const int64_t t128 = count_tiles(m, gs, ng, kShapes[2]);
-  const int64_t t6432 = count_tiles(m, gs, ng, kShapes[3]);
-  if (kmin >= 1024 && fills(t128)) {
-    p.shape = 2;
-    tiles = t128;
-  } else if (kmin >= 1024 && fills(t6432)) {
-    p.shape = 3;
-    tiles = t6432;
-  } else if (count_tiles(m, gs, ng, kShapes[0]) * 2 >= int64_t(cus) * 3) {
+  const int64_t units = std::max(cus, 1);
+  auto rounds = [](int64_t t, int64_t slots) { return double((t + slots - 1) / slots); };
+  if (kmin >= 1024) {
+    double best = tiles <= units ? 8.2 : 9.6 * rounds(tiles, 2 * units);
+    const struct { int shape; double us; } wide[] = {{3, 9.1}, {2, 16.5}};
+    for (const auto& w : wide) {
+      const int64_t t = count_tiles(m, gs, ng, kShapes[w.shape]);
+      const double us = w.us * rounds(t, units);
+      if (us < best) {
+        best = us;
+        p.shape = w.shape;
+      }
+    }
+    tiles = count_tiles(m, gs, ng, kShapes[p.shape]);
+  } else if (count_tiles(m, gs, ng, kShapes[0]) >= units) {
     p.shape = 0;
     tiles = count_tiles(m, gs, ng, kShapes[0]);
   }
-  // At most one workgroup per two units and long k: split k so that about two
+  // 32 x 32 tiles for at most half of the units and long k: split k so that about two
   // workgroups per unit each walk at least 8 stages. (With more tiles the
   // partials' extra traffic and second launch cost more than they save.)
   const int nk = (kmin + 63) / 64;
-  if (tiles * 2 <= int64_t(cus) && nk >= 16) {
+  if (p.shape == 1 && tiles * 2 <= int64_t(cus) && nk >= 16) {
     int64_t parts = (2 * int64_t(cus) + tiles / 2) / tiles;
     parts = std::min<int64_t>(parts, std::min(8, nk / 8));
     if (parts >= 2) {
@@ -538,8 +546,8 @@ extern "C" int wkv7_proj_grouped(int64_t m, const wkv7_proj_group* groups, int32
   float* ws = static_cast<float*>(workspace);
   hipStream_t s = as_stream(stream);
   if (p.shape == 0) return launch<64, 64, 2, 2, 4, 128>(m, groups, ngroups, p.parts, ws, s);
-  if (p.shape == 2) return launch<128, 64, 3, 2, 4, 128>(m, groups, ngroups, p.parts, ws, s);
-  if (p.shape == 3) return launch<64, 32, 4, 2, 2, 128>(m, groups, ngroups, p.parts, ws, s);
+  if (p.shape == 2) return launch<128, 64, 3, 8, 2, 128>(m, groups, ngroups, p.parts, ws, s);
+  if (p.shape == 3) return launch<64, 32, 4, 4, 2, 128>(m, groups, ngroups, p.parts, ws, s);
   return launch<32, 32, 4, 2, 2, 128>(m, groups, ngroups, p.parts, ws, s);
 }
 
@@ -561,7 +569,7 @@ extern "C" int wkv7_proj_grouped_noalloc(int64_t m, const wkv7_proj_group* group
   }
   hipStream_t s = as_stream(stream);
   if (p.shape == 0) return launch<64, 64, 2, 2, 4, 128>(m, groups, ngroups, p.parts, ws, s);
-  if (p.shape == 2) return launch<128, 64, 3, 2, 4, 128>(m, groups, ngroups, p.parts, ws, s);
-  if (p.shape == 3) return launch<64, 32, 4, 2, 2, 128>(m, groups, ngroups, p.parts, ws, s);
+  if (p.shape == 2) return launch<128, 64, 3, 8, 2, 128>(m, groups, ngroups, p.parts, ws, s);
+  if (p.shape == 3) return launch<64, 32, 4, 4, 2, 128>(m, groups, ngroups, p.parts, ws, s);
   return launch<32, 32, 4, 2, 2, 128>(m, groups, ngroups, p.parts, ws, s);
 }
