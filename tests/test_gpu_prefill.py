@@ -793,3 +793,61 @@ def test_all_layers_in_one_launch_equal_one_launch_each(dev, L, H, lens, y_dtype
         assert torch.equal(ys[layer][start:start + T], y)
         assert (ys[layer][:start] == 7).all() and (ys[layer][start + T:] == 7).all()
     assert torch.equal(wkv, ref)
+
+
+@pytest.mark.parametrize("y_dtype", [torch.bfloat16, torch.float32])
+def test_segment_chain_and_correct_against_float64(dev, y_dtype):
+    """The two combination kernels of the segmented prefill on random
+    matrices: H_out = H0 + Phi H_in over 0, 1 and 3 segments, and y = y0 + q
+    H_in for token blocks around the 16 tokens of a wave (and one without a
+    correction). The products take q and H_in as bf16 hi + lo parts, each
+    within 2^-18 of its value, without the lo x lo term (2^-18): 2^-16.4 of
+    the summed magnitudes, plus fp32 accumulation of 64 terms."""
+    from wkvm_amd import _lib
+
+    lib, H, N = _lib.load(), 3, 64
+    stream = torch.cuda.current_stream().cuda_stream
+    g = synthetic.make_generator(61, dev)
+    rnd = lambda *s: torch.randn(s, generator=g, device=dev)  # noqa: E731
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    pool, alt, nsegs = rnd(4, H, N, N), rnd(8, H, N, N) * 0.1, 4
+    hin = torch.zeros((nsegs, H, N, N), device=dev)
+    seq_tab, seg_tab = [1, 0, 1, 2, 1, 3, 3, 4, 0], [0, 1, 2, 3, 4, 5, 6, 7]
+    ref = pool.double()
+    want = torch.zeros_like(hin, dtype=torch.float64)
+    for slot, first, count in (seq_tab[i:i + 3] for i in (0, 3, 6)):
+        for s in range(first, first + count):
+            want[s] = ref[slot]
+            ref[slot] = alt[2 * s].double() + alt[2 * s + 1].double() @ ref[slot]
+    d_seq, d_seg = i32(seq_tab), i32(seg_tab)
+    rc = lib.wkv7_segment_chain(pool.data_ptr(), 4, H, alt.data_ptr(), 8, d_seq.data_ptr(), 3,
+                                d_seg.data_ptr(), nsegs, hin.data_ptr(), stream)
+    assert rc == 0
+    torch.cuda.synchronize()
+    assert U.rel_l2(U.f64(hin), want.cpu().numpy()) <= 64 * 2.0**-24
+    assert U.rel_l2(U.f64(pool), ref.cpu().numpy()) <= 64 * 2.0**-24
+
+    counts = [(1, 0), (15, 1), (16, 2), (17, 3), (64, 0), (33, -1), (63, 3)]
+    T = sum(c for c, _ in counts)
+    blk, at = [], 0
+    for c, s in counts:
+        blk += [at, c, s]
+        at += c
+    y0, q, d_blk = rnd(T, H, N), rnd(T, H, N), i32(blk)
+    y = torch.empty((T, H, N), dtype=y_dtype, device=dev)
+    rc = lib.wkv7_segment_correct(T, H, y0.data_ptr(), q.data_ptr(), d_blk.data_ptr(),
+                                  len(counts), hin.data_ptr(), nsegs, y.data_ptr(),
+                                  _lib.WKV7_Y_F32 if y_dtype == torch.float32 else
+                                  _lib.WKV7_Y_BF16, stream)
+    assert rc == 0
+    torch.cuda.synchronize()
+    exact, size = y0.double(), y0.abs().double()
+    for i, (c, s) in enumerate(counts):
+        if s >= 0:
+            t = slice(blk[3 * i], blk[3 * i] + c)
+            exact[t] += torch.einsum("thk,hkv->thv", q[t].double(), hin[s].double())
+            size[t] += torch.einsum("thk,hkv->thv", q[t].abs().double(), hin[s].abs().double())
+    bar = size * (2.0**-16.4 + 64 * 2.0**-24)
+    if y_dtype == torch.bfloat16:
+        bar = bar + exact.abs() * 2.0**-8
+    assert ((y.double() - exact).abs() <= bar).all()

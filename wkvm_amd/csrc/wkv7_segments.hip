@@ -8,9 +8,9 @@
 // entering segment g:
 //   H_out = H0_g + Phi_g H_in          (wkv7_segment_chain, in segment order)
 //   y_g   = y0_g + q_g H_in            (wkv7_segment_correct, all tokens at once)
-// Both in fp32; state matrices use the pool layout [j][i] (key j, value i),
+// Both accumulate in fp32; state matrices use the pool layout [j][i] (key j, value i),
 // on which Phi acts from the left.
-#include "wkv7_common.h"
+#include "wkv7_mfma.h"
 
 namespace wkv7 {
 namespace {
@@ -18,119 +18,136 @@ namespace {
 constexpr int kCombThreads = 256;
 constexpr int kMat = kHead * kHead;  // floats per 64 x 64 head matrix
 
-// One (sequence, head) per workgroup; thread t owns row j = t / 4 and the 16
-// columns 16 (t % 4) .. + 15 of the 64 x 64 products.
+// A quarter (16 value columns) of one (sequence, head) per workgroup; thread t
+// owns row j = t / 4 and the columns 16 q + 4 (t % 4) .. + 3 of the products.
+// The columns are independent, and one workgroup per head left most units
+// idle: three segments of 32 heads 20 us whole, 8 us in quarters.
+constexpr int kChainSplit = 4;
 __global__ __launch_bounds__(kCombThreads) void segment_chain_kernel(
     float* __restrict__ wkv, int64_t num_rows, int H, const float* __restrict__ alt,
     int64_t alt_rows, const int32_t* __restrict__ seq_tab, int nseq,
     const int32_t* __restrict__ seg_tab, int nsegs, float* __restrict__ hin) {
-  __shared__ float4 cur[kMat / 4];  // H_in, row-major [m][c]
-  const int64_t s = blockIdx.x / H;
-  const int64_t head = blockIdx.x - s * H;
+  __shared__ float4 cur[kHead][4];  // H_in, these columns
+  const int64_t item = blockIdx.x / kChainSplit;
+  const int64_t s = item / H;
+  const int64_t head = item - s * H;
   if (s >= nseq) return;
   const int64_t slot = seq_tab[3 * s];
   const int first = seq_tab[3 * s + 1], count = seq_tab[3 * s + 2];
   if (slot < 0 || slot >= num_rows || first < 0 || count < 0 || first + count > nsegs) return;
-  float4* state = reinterpret_cast<float4*>(wkv + (slot * H + head) * kMat);
-  const int t = threadIdx.x;
-  for (int i = t; i < kMat / 4; i += kCombThreads) cur[i] = state[i];
-  __syncthreads();
-  const int j = t >> 2, c4 = (t & 3) * 4;  // row j, float4 columns c4 .. c4 + 3
+  const int j = threadIdx.x >> 2, c = threadIdx.x & 3;
+  const int at = j * 16 + 4 * int(blockIdx.x % kChainSplit) + c;  // this thread's float4
+  float4* state = reinterpret_cast<float4*>(wkv + (slot * H + head) * kMat) + at;
+  float4 h = *state;
   for (int n = 0; n < count; ++n) {
     const int seg = first + n;
     const int64_t row_main = seg_tab[2 * seg], row_phi = seg_tab[2 * seg + 1];
-    float4* hout = reinterpret_cast<float4*>(hin + (int64_t(seg) * H + head) * kMat);
-    for (int i = t; i < kMat / 4; i += kCombThreads) hout[i] = cur[i];
+    reinterpret_cast<float4*>(hin + (int64_t(seg) * H + head) * kMat)[at] = h;
     const bool ok = row_main >= 0 && row_main < alt_rows && row_phi >= 0 && row_phi < alt_rows;
-    float4 acc[4];
-    if (ok) {
-      const float4* phi = reinterpret_cast<const float4*>(alt + (row_phi * H + head) * kMat);
-      const float4* h0 = reinterpret_cast<const float4*>(alt + (row_main * H + head) * kMat);
+    if (!ok) continue;  // uniform
+    cur[j][c] = h;
+    __syncthreads();
+    const float4* phi = reinterpret_cast<const float4*>(alt + (row_phi * H + head) * kMat);
+    h = reinterpret_cast<const float4*>(alt + (row_main * H + head) * kMat)[at];
+    for (int m4 = 0; m4 < 16; ++m4) {
+      const float4 p = phi[j * 16 + m4];
+      const float pv[4] = {p.x, p.y, p.z, p.w};
 #pragma unroll
-      for (int q = 0; q < 4; ++q) acc[q] = h0[j * 16 + c4 + q];
-      for (int m4 = 0; m4 < 16; ++m4) {
-        const float4 p = phi[j * 16 + m4];
-        const float pv[4] = {p.x, p.y, p.z, p.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int m = 4 * m4 + e;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const float4 hv = cur[m * 16 + c4 + q];
-            acc[q].x = fmaf(pv[e], hv.x, acc[q].x);
-            acc[q].y = fmaf(pv[e], hv.y, acc[q].y);
-            acc[q].z = fmaf(pv[e], hv.z, acc[q].z);
-            acc[q].w = fmaf(pv[e], hv.w, acc[q].w);
-          }
-        }
+      for (int e = 0; e < 4; ++e) {
+        const float4 hv = cur[4 * m4 + e][c];
+        h.x = fmaf(pv[e], hv.x, h.x);
+        h.y = fmaf(pv[e], hv.y, h.y);
+        h.z = fmaf(pv[e], hv.z, h.z);
+        h.w = fmaf(pv[e], hv.w, h.w);
       }
     }
     __syncthreads();  // every thread has read cur
-    if (ok) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) cur[j * 16 + c4 + q] = acc[q];
-    }
-    __syncthreads();
   }
-  for (int i = t; i < kMat / 4; i += kCombThreads) state[i] = cur[i];
+  *state = h;
 }
 
-// One block of at most 64 tokens of one head per workgroup; thread t owns
-// token t / 4 of the block and the 16 value columns 16 (t % 4) .. + 15.
+// One block of at most 64 tokens of one head per workgroup, 16 tokens per
+// wave: y^T = y0^T + H_in^T q^T on the matrix cores, H_in and q as bf16 hi + lo
+// (three products per term, ~2^-16 relative) on the fp32 y0 as the accumulator.
+// It moves 564 bytes per token-head and runs near that (16384 tokens x 32
+// heads); as 64 fp32 multiply-adds per value out of LDS it read 16 KiB of LDS
+// per token and took 88 us.
 template <bool kF32Out>
 __global__ __launch_bounds__(kCombThreads) void segment_correct_kernel(
     int64_t total_tokens, int H, const float* __restrict__ y0, const float* __restrict__ q,
     const int32_t* __restrict__ blk_tab, int nblk, const float* __restrict__ hin, int nsegs,
     void* __restrict__ y) {
-  __shared__ float4 mat[kMat / 4];
+  __shared__ __align__(16) uint16_t hs[2][kHead * kPR];  // H_in hi, lo: [key][value column]
   const int64_t blk = blockIdx.x / H;
   const int64_t head = blockIdx.x - blk * H;
   if (blk >= nblk) return;
   const int64_t tok0 = blk_tab[3 * blk];
   const int cnt = blk_tab[3 * blk + 1], seg = blk_tab[3 * blk + 2];
   const bool corr = seg >= 0 && seg < nsegs;
-  const int t = threadIdx.x;
-  if (corr) {
-    const float4* src = reinterpret_cast<const float4*>(hin + (int64_t(seg) * H + head) * kMat);
-    for (int i = t; i < kMat / 4; i += kCombThreads) mat[i] = src[i];
-  }
-  __syncthreads();
-  const int ti = t >> 2, c4 = (t & 3) * 4;
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int ti = 16 * int(threadIdx.x >> 6) + li;
   const int64_t tok = tok0 + ti;
-  if (ti >= cnt || tok < 0 || tok >= total_tokens) return;
+  const bool mine = ti < cnt && tok >= 0 && tok < total_tokens;
   const int64_t base = (tok * H + head) * kHead;
-  const float4* y0r = reinterpret_cast<const float4*>(y0 + base);
-  float4 acc[4];
+  // lane: token li, value columns 16 ct + 4 lg .. + 3 of every tile ct
+  f32x4 acc[4] = {}, qv[2][2] = {};
+  if (mine) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) acc[e] = y0r[c4 + e];
-  if (corr) {
-    const float4* qr = reinterpret_cast<const float4*>(q + base);
-    for (int m4 = 0; m4 < 16; ++m4) {
-      const float4 qv = qr[m4];
-      const float qs[4] = {qv.x, qv.y, qv.z, qv.w};
+    for (int ct = 0; ct < 4; ++ct)
+      acc[ct] = __builtin_nontemporal_load(
+          reinterpret_cast<const f32x4*>(y0 + base + 16 * ct + 4 * lg));
+    if (corr) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int m = 4 * m4 + e;
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const float4 hv = mat[m * 16 + c4 + u];
-          acc[u].x = fmaf(qs[e], hv.x, acc[u].x);
-          acc[u].y = fmaf(qs[e], hv.y, acc[u].y);
-          acc[u].z = fmaf(qs[e], hv.z, acc[u].z);
-          acc[u].w = fmaf(qs[e], hv.w, acc[u].w);
-        }
-      }
+        for (int i = 0; i < 2; ++i)
+          qv[kb][i] = __builtin_nontemporal_load(
+              reinterpret_cast<const f32x4*>(q + base + 32 * kb + 8 * lg + 4 * i));
     }
   }
-  if (kF32Out) {
-    float4* yr = reinterpret_cast<float4*>(static_cast<float*>(y) + base);
+  if (corr) {  // uniform
+    const Neg n = neg_consts();
+    const f32x4* src = reinterpret_cast<const f32x4*>(hin + (int64_t(seg) * H + head) * kMat);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) yr[c4 + e] = acc[e];
-  } else {
-    uint2* yr = reinterpret_cast<uint2*>(static_cast<uint16_t*>(y) + base);
+    for (int i = 0; i < kMat / 4 / kCombThreads; ++i) {
+      const int at = kCombThreads * i + threadIdx.x;
+      uint2 hi, lo;
+      pack_split(src[at], hi, lo, n);
+      const int off = rk_off(at >> 4, 4 * (at & 15));
+      *reinterpret_cast<uint2*>(&hs[0][off]) = hi;
+      *reinterpret_cast<uint2*>(&hs[1][off]) = lo;
+    }
+    uint4 qh[2], ql[2];
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      yr[c4 + e] = make_uint2(pack_bf16(acc[e].x, acc[e].y), pack_bf16(acc[e].z, acc[e].w));
+    for (int kb = 0; kb < 2; ++kb) {
+      uint2 h0, l0, h1, l1;
+      pack_split(qv[kb][0], h0, l0, n);
+      pack_split(qv[kb][1], h1, l1, n);
+      qh[kb] = make_uint4(h0.x, h0.y, h1.x, h1.y);
+      ql[kb] = make_uint4(l0.x, l0.y, l1.x, l1.y);
+    }
+    __syncthreads();
+    // A operand H_in^T: value column 16 ct + li at keys 32 kb + 8 lg .. + 7
+    auto tile = [&](const uint16_t* m, int ct, int kb) {
+      const int r = 32 * kb + 8 * lg + (li >> 2), c = 16 * ct + 4 * (li & 3);
+      const uint2 a = ld_tr(m + rk_off(r, c)), b = ld_tr(m + rk_off(r + 4, c));
+      return make_uint4(a.x, a.y, b.x, b.y);
+    };
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+        acc[ct] = mma32x3(tile(hs[0], ct, kb), tile(hs[1], ct, kb), qh[kb], ql[kb], acc[ct]);
+  }
+  if (!mine) return;
+#pragma unroll
+  for (int ct = 0; ct < 4; ++ct) {
+    const int64_t o = base + 16 * ct + 4 * lg;
+    if constexpr (kF32Out)
+      *reinterpret_cast<f32x4*>(static_cast<float*>(y) + o) = acc[ct];
+    else
+      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(y) + o) =
+          make_uint2(pack_bf16(acc[ct][0], acc[ct][1]), pack_bf16(acc[ct][2], acc[ct][3]));
   }
 }
 
@@ -151,7 +168,7 @@ extern "C" int wkv7_segment_chain(float* wkv_layer, int64_t num_rows, int32_t H,
     return WKV7_ERR_ARG;
   if (!aligned16(wkv_layer) || (nsegs > 0 && (!aligned16(state_alt) || !aligned16(hin))))
     return WKV7_ERR_SHAPE;
-  const int64_t blocks = int64_t(nseq) * H;
+  const int64_t blocks = int64_t(nseq) * H * kChainSplit;
   if (blocks > int64_t(0x7fffffff)) return WKV7_ERR_ARG;
   segment_chain_kernel<<<unsigned(blocks), kCombThreads, 0, as_stream(stream)>>>(
       wkv_layer, num_rows, H, state_alt, alt_rows, seq_tab, nseq, seg_tab, nsegs, hin);
