@@ -197,3 +197,35 @@ def test_every_tile_shape_of_long_k(dev, M):
                       _rand((n,), gen, dev), act))
     for y, (x, w, b, act) in zip(ops.proj_grouped(prods), prods):
         _assert_within_one_ulp(y, _exact(x, w, b, act))
+
+
+@pytest.mark.parametrize("M", [1, 15, 16, 17])
+@pytest.mark.parametrize("ks,ns", [((32, 96, 256, 512), (2048, 72, 1, 2040)),
+                                   ((768, 2080, 1056), (768, 40, 1000)),
+                                   ((4096,), (2048,)),
+                                   ((2048, 2048), (2049, 2048))])
+def test_few_rows(dev, M, ks, ns):
+    """Either side of the row count, the longest short k and the column count where
+    the kernel of one row tile hands over; k of one to nine chunks per wave, half
+    chunks, ragged n; the rows around y stay as they were."""
+    gen = torch.Generator().manual_seed(67)
+    prods, outs, bufs = [], [], []
+    for i, (k, n) in enumerate(zip(ks, ns)):
+        prods.append((_rand((M, k), gen, dev), _rand((n, k), gen, dev, 1 / math.sqrt(k)),
+                      _rand((n,), gen, dev) if i % 2 else None, (None, "tanh", "sigmoid")[i % 3]))
+        bufs.append(torch.full((M + 2, n + 3), 7.0, dtype=torch.bfloat16, device=dev))
+        outs.append(bufs[-1][1:-1, :n])
+    ops.proj_grouped(prods, outs=outs)
+    for y, buf, (x, w, b, act) in zip(outs, bufs, prods):
+        _assert_within_one_ulp(y, _exact(x, w, b, act))
+        assert bool((buf[0] == 7.0).all()) and bool((buf[-1] == 7.0).all())
+        assert bool((buf[:, y.shape[1]:] == 7.0).all())
+
+
+def test_split_k_above_the_row_tile(dev):
+    """17 rows of long k and few columns: the k split of the tiled kernel."""
+    gen = torch.Generator().manual_seed(71)
+    x, w = _rand((17, 2080), gen, dev), _rand((1000, 2080), gen, dev, 1 / math.sqrt(2080))
+    b = _rand((1000,), gen, dev)
+    (y,) = ops.proj_grouped([(x, w, b, "tanh")])
+    _assert_within_one_ulp(y, _exact(x, w, b, "tanh"))

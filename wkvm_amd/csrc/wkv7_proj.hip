@@ -24,7 +24,8 @@
 // XCDs in contiguous runs so that each XCD's L2 keeps the x rows it
 // re-reads. With few tiles and long k, k can be split over several
 // workgroups per tile (fp32 partials in a caller-provided workspace, summed
-// in part order by proj_reduce_kernel).
+// in part order by proj_reduce_kernel). Up to 16 rows have a kernel of their own
+// (proj_thin_kernel) where it is the faster one.
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -341,6 +342,72 @@ __global__ __launch_bounds__(256) void proj_reduce_kernel(const ProjArgs args) {
   G.y[row * G.ldy + col] = f32_to_bf16(activate(sum + bias, G.act));
 }
 
+// One row tile (m <= 16): a 16-column tile of a product by one workgroup, its
+// k dealt to NW waves in 64-wide chunks (wave w: chunks w, w + NW, ..), so that
+// the workgroup reads contiguous bytes of each weight row. Every operand goes
+// from memory straight to registers and up to four chunks of a wave are in
+// flight at once: with few rows there is nothing to share through LDS, and what
+// bounds the launch is the latency of the weights' one pass from memory, which
+// a ring with a barrier per stage pays several times. The waves' fp32 partial
+// tiles are summed through LDS in wave order. 16 rows, us per launch in a HIP
+// graph over distinct weights, before (32 x 32 tiles, k split) and now: LoRA
+// up-projections 4.3 -> 3.6, o_proj 8.0 -> 6.7 (8.6 MB); hidden size 768: first
+// stage 5.4 -> 4.6, o_proj 5.0 -> 4.0. Slower: 32 columns per workgroup (o_proj
+// 8.7: half of the workgroups), non-temporal weight loads (7.2), 16 waves.
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void proj_thin_kernel(const ProjArgs args) {
+  __shared__ f32x4 red[NW][64];
+  const int bid = int(blockIdx.x);
+  int g = 0;
+  while (g + 1 < args.ngroups && bid >= args.tile_end[g]) ++g;
+  const wkv7_proj_group& G = args.g[g];
+  const int n0 = (bid - (g ? args.tile_end[g - 1] : 0)) * 16;
+  const int M = int(args.m), N = G.n, K = G.k;
+  const int t = threadIdx.x, lane = t & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  // A: 16 rows of w, B: 16 rows of x (rows past the end repeat the last one and
+  // are not stored); the accumulator holds columns n0 + 4 lg .. + 3 of row li.
+  const uint16_t* wp = G.w + int64_t(min(n0 + li, N - 1)) * G.ldw + 8 * lg;
+  const uint16_t* xp = G.x + int64_t(min(li, M - 1)) * G.ldx + 8 * lg;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  // U chunks of this wave from chunk c on. Only the last chunk of all can be
+  // half a chunk wide: its second half re-reads the first and is left out.
+  auto chunks = [&](int c, auto u_c) {
+    constexpr int U = decltype(u_c)::value;
+    uint4 wf[U][2], xf[U][2];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k0 = 64 * (c + u * NW), k1 = k0 + 32 < K ? k0 + 32 : k0;
+      wf[u][0] = *reinterpret_cast<const uint4*>(wp + k0);
+      wf[u][1] = *reinterpret_cast<const uint4*>(wp + k1);
+      xf[u][0] = *reinterpret_cast<const uint4*>(xp + k0);
+      xf[u][1] = *reinterpret_cast<const uint4*>(xp + k1);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      acc = mma(wf[u][0], xf[u][0], acc);
+      if (64 * (c + u * NW) + 32 < K) acc = mma(wf[u][1], xf[u][1], acc);
+    }
+  };
+  const int nc = (K + 63) / 64;
+  int c = wave;
+  for (; c + 3 * NW < nc; c += 4 * NW) chunks(c, std::integral_constant<int, 4>{});
+  if (c + 2 * NW < nc) chunks(c, std::integral_constant<int, 3>{});
+  else if (c + NW < nc) chunks(c, std::integral_constant<int, 2>{});
+  else if (c < nc) chunks(c, std::integral_constant<int, 1>{});
+  red[wave][lane] = acc;
+  __syncthreads();
+  if (t >= 256) return;  // thread t: row t / 16, column t % 16 of the tile
+  const int row = t >> 4, col = t & 15;
+  if (row >= M || n0 + col >= N) return;
+  const float* part = reinterpret_cast<const float*>(&red[0][(col >> 2) * 16 + row]) + (col & 3);
+  float sum = 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) sum += part[w * 64 * 4];
+  const float bias = G.bias ? bf16_to_f32(G.bias[n0 + col]) : 0.f;
+  G.y[row * G.ldy + n0 + col] = f32_to_bf16(activate(sum + bias, G.act));
+}
+
 struct TileShape {
   int bm, bn;
 };
@@ -390,6 +457,22 @@ int launch(int64_t m, const wkv7_proj_group* gs, int ng, int parts, float* ws, h
   return launch_status();
 }
 
+template <int NW>
+int launch_thin(int64_t m, const wkv7_proj_group* gs, int ng, hipStream_t s) {
+  ProjArgs args{};
+  args.m = m;
+  args.ngroups = ng;
+  int64_t end = 0;
+  for (int i = 0; i < ng; ++i) {
+    args.g[i] = gs[i];
+    end += (int64_t(gs[i].n) + 15) / 16;
+    if (end > int64_t(0x7fffffff)) return WKV7_ERR_ARG;
+    args.tile_end[i] = int32_t(end);
+  }
+  proj_thin_kernel<NW><<<unsigned(end), 64 * NW, 0, s>>>(args);
+  return launch_status();
+}
+
 // Tile shape and k split for a launch (the same decision for the workspace
 // query and the launch).
 struct Plan {
@@ -398,6 +481,24 @@ struct Plan {
   size_t ws_bytes;
 };
 
+// One row tile: the thin kernel for few column tiles, where it has no second
+// launch, and for short k. Not for many column tiles of long k: every one
+// re-reads all of x (1.5B first stage of 16 rows, 407 workgroups, 12.2 us
+// against 9.4 in 32 x 32 tiles; o_proj of the 7B shape, 256, 12.2 against 13.5).
+// Its waves: 8 for long k, 4 where k has few chunks (LoRA up-projections of the
+// 7B shape 5.2 against 6.4 us).
+constexpr int kThinRows = 16, kThinShortK = 512;
+
+int thin_waves(int64_t m, const wkv7_proj_group* gs, int ng, int cus) {
+  if (m > kThinRows) return 0;
+  int kmax = 0;
+  for (int i = 0; i < ng; ++i) kmax = std::max(kmax, gs[i].k);
+  if (kmax <= kThinShortK) return 4;
+  return count_tiles(m, gs, ng, kShapes[1]) * 2 <= int64_t(cus) ? 8 : 0;
+}
+
+// The plan of the tiled kernel (at 16 rows or fewer the thin one may run in its
+// place, and then leaves the workspace alone).
 Plan make_plan(int64_t m, const wkv7_proj_group* gs, int ng, int cus) {
   int kmin = gs[0].k;
   int64_t cols = 0;
@@ -450,6 +551,14 @@ Plan make_plan(int64_t m, const wkv7_proj_group* gs, int ng, int cus) {
     }
   }
   return p;
+}
+
+int launch_plan(int64_t m, const wkv7_proj_group* gs, int ng, const Plan& p, float* ws,
+                hipStream_t s) {
+  if (p.shape == 0) return launch<64, 64, 2, 2, 4, 128>(m, gs, ng, p.parts, ws, s);
+  if (p.shape == 2) return launch<128, 64, 3, 8, 2, 128>(m, gs, ng, p.parts, ws, s);
+  if (p.shape == 3) return launch<64, 32, 4, 4, 2, 128>(m, gs, ng, p.parts, ws, s);
+  return launch<32, 32, 4, 2, 2, 128>(m, gs, ng, p.parts, ws, s);
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -539,16 +648,15 @@ extern "C" int wkv7_proj_grouped(int64_t m, const wkv7_proj_group* groups, int32
   int cus = 0;
   const int drc = device_cus(&cus);
   if (drc != WKV7_OK) return drc;
+  const int waves = thin_waves(m, groups, ngroups, cus);
+  if (waves == 4) return launch_thin<4>(m, groups, ngroups, as_stream(stream));
+  if (waves == 8) return launch_thin<8>(m, groups, ngroups, as_stream(stream));
   Plan p = make_plan(m, groups, ngroups, cus);
   // without (enough) workspace every tile's workgroup covers all of k
   if (p.parts > 1 && (!workspace || workspace_bytes < p.ws_bytes || !aligned16(workspace)))
     p.parts = 1;
   float* ws = static_cast<float*>(workspace);
-  hipStream_t s = as_stream(stream);
-  if (p.shape == 0) return launch<64, 64, 2, 2, 4, 128>(m, groups, ngroups, p.parts, ws, s);
-  if (p.shape == 2) return launch<128, 64, 3, 8, 2, 128>(m, groups, ngroups, p.parts, ws, s);
-  if (p.shape == 3) return launch<64, 32, 4, 4, 2, 128>(m, groups, ngroups, p.parts, ws, s);
-  return launch<32, 32, 4, 2, 2, 128>(m, groups, ngroups, p.parts, ws, s);
+  return launch_plan(m, groups, ngroups, p, ws, as_stream(stream));
 }
 
 extern "C" int wkv7_proj_grouped_noalloc(int64_t m, const wkv7_proj_group* groups,
@@ -559,6 +667,9 @@ extern "C" int wkv7_proj_grouped_noalloc(int64_t m, const wkv7_proj_group* group
   int cus = 0;
   const int drc = device_cus(&cus);
   if (drc != WKV7_OK) return drc;
+  const int waves = thin_waves(m, groups, ngroups, cus);
+  if (waves == 4) return launch_thin<4>(m, groups, ngroups, as_stream(stream));
+  if (waves == 8) return launch_thin<8>(m, groups, ngroups, as_stream(stream));
   const Plan p = make_plan(m, groups, ngroups, cus);
   float* ws = nullptr;
   if (p.parts > 1) {
@@ -567,9 +678,5 @@ extern "C" int wkv7_proj_grouped_noalloc(int64_t m, const wkv7_proj_group* group
     const int src = scratch_address(&ws);
     if (src != WKV7_OK) return src;
   }
-  hipStream_t s = as_stream(stream);
-  if (p.shape == 0) return launch<64, 64, 2, 2, 4, 128>(m, groups, ngroups, p.parts, ws, s);
-  if (p.shape == 2) return launch<128, 64, 3, 8, 2, 128>(m, groups, ngroups, p.parts, ws, s);
-  if (p.shape == 3) return launch<64, 32, 4, 4, 2, 128>(m, groups, ngroups, p.parts, ws, s);
-  return launch<32, 32, 4, 2, 2, 128>(m, groups, ngroups, p.parts, ws, s);
+  return launch_plan(m, groups, ngroups, p, ws, as_stream(stream));
 }
