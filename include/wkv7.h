@@ -314,6 +314,24 @@ int wkv7_slot_copy(void *dst, int64_t dst_outer_stride, int64_t dst_slot_stride,
                    int64_t outer, int64_t row_bytes, int32_t n, void *stream);
 
 /*
+ * A fork within one or two slot tensors at once: row dst_ids[p] of every outer
+ * block becomes a copy of row src_ids[p], p = 0 .. n-1 (strides in bytes). The
+ * ids are host arrays, read before the call returns (nothing is uploaded); one
+ * outside [0, rows) is WKV7_ERR_ARG and nothing is copied. Base, strides and
+ * row_bytes are multiples of 16 (else WKV7_ERR_SHAPE: use wkv7_slot_copy).
+ * Replaces the copy that StateArena.fork leaves to the runner
+ * (wkvm/core/arena.py:82-93) for both state families together; preconditions
+ * as for wkv7_slot_copy.
+ */
+struct wkv7_slot_family {
+    void *base;
+    int64_t outer_stride, slot_stride, rows, outer, row_bytes;
+    const int32_t *dst_ids, *src_ids;
+};
+int wkv7_slot_fork(const struct wkv7_slot_family *families, int32_t nfamilies, int32_t n,
+                   void *stream);
+
+/*
  * Zero slot rows (admission reset: zero state == empty prefix).
  * Replaces RWKV7StateBank.zero_slots (wkvm/runner/state.py:50-54). Uses a fill
  * kernel, not a memset node, so it is safe inside captured HIP graphs.

@@ -181,3 +181,38 @@ def test_fork_7b_shape_128_slots(dev):
     assert torch.equal(wkv[:, 1:1025].sum(dim=(2, 3, 4)), keep)
     del wkv, shift
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("pairs", [1, 2, 128, 129, 300])
+@pytest.mark.parametrize("heads,head_dim", [(1, 64), (3, 64), (33, 64), (1, 2), (3, 1)])
+def test_fork_families_with_their_own_ids(dev, pairs, heads, head_dim):
+    """One launch for both families up to its pair limit and beyond, different ids per
+    family, rows of less than a tile to many tiles and a remainder; rows that
+    are no 16-byte vectors take the copy kernel."""
+    layout = RWKV7StateLayout(n_layer=2, hidden_size=heads * head_dim, num_heads=heads,
+                              head_dim=head_dim, head_v_dim=head_dim, dtype=torch.bfloat16)
+    slots = 2 * pairs + 3
+    bank = RWKV7StateBank(layout, num_slots=slots, device=dev)
+    g = torch.Generator().manual_seed(pairs)
+    bank.wkv.normal_()
+    bank.shift.normal_()
+    ids = {f: (torch.randperm(slots, generator=g) + 1).tolist() for f in ("wkv", "shift")}
+    src = [{f: ids[f][p // 2] for f in ids} for p in range(pairs)]
+    dst = [{f: ids[f][pairs + p] for f in ids} for p in range(pairs)]
+    wkv, shift = bank.wkv.clone(), bank.shift.clone()
+    wkv[:, [d["wkv"] for d in dst]] = wkv[:, [s["wkv"] for s in src]]
+    shift[:, :, [d["shift"] for d in dst]] = shift[:, :, [s["shift"] for s in src]]
+    bank.fork_slots(src, dst)
+    assert torch.equal(bank.wkv, wkv)
+    assert torch.equal(bank.shift, shift)
+
+
+def test_fork_copies_nothing_when_a_family_is_refused(dev):
+    bank = _small_bank(dev)
+    bank.wkv.normal_()
+    before = bank.wkv.clone()
+    with pytest.raises(ValueError, match="out of range"):
+        bank.fork_slots([{"wkv": 1, "shift": 1}], [{"wkv": 2, "shift": 5}])
+    assert torch.equal(bank.wkv, before)
+    bank.fork_slots([], [])
+    assert torch.equal(bank.wkv, before)

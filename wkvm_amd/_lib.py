@@ -54,6 +54,12 @@ class ProjGroup(ctypes.Structure):
                 ("reserved", _i32)]
 
 
+class SlotFamily(ctypes.Structure):
+    """struct wkv7_slot_family of include/wkv7.h."""
+    _fields_ = [("base", _vp), ("outer_stride", _i64), ("slot_stride", _i64), ("rows", _i64),
+                ("outer", _i64), ("row_bytes", _i64), ("dst_ids", _vp), ("src_ids", _vp)]
+
+
 # name -> (restype, argtypes); must match include/wkv7.h.
 SIGNATURES = {
     "wkv7_abi_version": (ctypes.c_int, []),
@@ -82,6 +88,7 @@ SIGNATURES = {
         _i64, _i32, _vp, _vp, _vp, _i32, _vp, _i32, _vp, _i32, _vp]),
     "wkv7_slot_copy": (ctypes.c_int, [
         _vp, _i64, _i64, _i64, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _i32, _vp]),
+    "wkv7_slot_fork": (ctypes.c_int, [_vp, _i32, _i32, _vp]),
     "wkv7_slot_zero": (ctypes.c_int, [_vp, _i64, _i64, _i64, _vp, _i64, _i64, _i32, _vp]),
     "wkv7_slot_transfer": (ctypes.c_int, [_i32, _vp, _vp, _i64, _i64, _i64, _i32, _i64, _i64,
                                          _vp, _sz, _vp]),

@@ -81,10 +81,9 @@ class RWKV7StateBank:
         bit-exact. Destinations must be distinct fresh slots (not sources)."""
         if len(src_batch) != len(dst_batch):
             raise ValueError("src_batch and dst_batch length mismatch")
-        ops.slot_copy(self.wkv, ops.ids_list(dst_batch, "wkv"), self.wkv,
-                      ops.ids_list(src_batch, "wkv"), slot_dim=1)
-        ops.slot_copy(self.shift, ops.ids_list(dst_batch, "shift"), self.shift,
-                      ops.ids_list(src_batch, "shift"), slot_dim=2)
+        ops.slot_fork([(t, slot_dim, ops.ids_list(dst_batch, family),
+                        ops.ids_list(src_batch, family))
+                       for t, slot_dim, family in ((self.wkv, 1, "wkv"), (self.shift, 2, "shift"))])
 
     # -- gather / scatter (kept for cache-staging callers) ---------------------------
 
