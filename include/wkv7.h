@@ -193,6 +193,17 @@ int wkv7_decode_layers(float *wkv, int64_t layer_stride, int32_t layers, int64_t
                        int32_t H, const int32_t *slot_ids, const int32_t *row_order, int32_t B,
                        const struct wkv7_layer_io *io, int32_t y_dtype, float scale,
                        void *stream);
+/*
+ * wkv7_decode_layers with the slot ids in a host array, read before the call
+ * returns (nothing is uploaded), for at most WKV7_DECODE_MAX_HOST_IDS rows; an id
+ * outside [0, num_rows) or given twice is WKV7_ERR_ARG. Rows are visited in
+ * slot order.
+ */
+#define WKV7_DECODE_MAX_HOST_IDS 256
+int wkv7_decode_layers_ids(float *wkv, int64_t layer_stride, int32_t layers, int64_t num_rows,
+                           int32_t H, const int32_t *host_ids, int32_t B,
+                           const struct wkv7_layer_io *io, int32_t y_dtype, float scale,
+                           void *stream);
 int wkv7_prefill_layers(float *wkv, int64_t layer_stride, int32_t layers, int64_t num_rows,
                         int32_t H, const int32_t *slot_ids, const int32_t *cu_seqlens,
                         const int32_t *seq_order, int32_t nseq, int64_t total_tokens,

@@ -464,3 +464,28 @@ def test_all_layers_in_one_launch_equal_one_launch_each(dev, L, B, H, y_dtype):
         ops.wkv7_decode_layers(wkv, ids, xs[1:])
     with pytest.raises(ValueError, match="bfloat16"):
         ops.wkv7_decode_layers(wkv, ids, [(x[0].float(), *x[1:]) for x in xs])
+
+
+@pytest.mark.parametrize("B", [1, 7, 255, 256, 257])
+@pytest.mark.parametrize("layers", [1, 33])
+def test_host_ids_equal_device_ids(dev, B, layers):
+    """Ids in the kernel arguments (up to 256 rows, one launch per 32 layers) give the
+    bits of uploaded ones, in any order of the slots."""
+    H, rows = 1, 300
+    g = torch.Generator().manual_seed(B)
+    ids = torch.randperm(rows, generator=g)[:B].tolist()
+    gen = torch.Generator(device=dev).manual_seed(B)
+    xs = [[torch.randn((B, H, 64), generator=gen, device=dev).to(torch.bfloat16) * 0.3
+           for _ in range(6)] for _ in range(layers)]
+    for x in xs:
+        x[1].sigmoid_().neg_()
+    wkv = torch.randn((layers, rows, H, 64, 64), generator=gen, device=dev)
+    want = wkv.clone()
+    dev_ids, order = ops.decode_plan(ids, rows, torch.device(wkv.device))
+    ys_want = ops.wkv7_decode_layers(want, dev_ids, xs, row_order=order)
+    ys = ops.wkv7_decode_layers(wkv, ids, xs)
+    assert torch.equal(wkv, want)
+    assert all(torch.equal(a, b) for a, b in zip(ys, ys_want))
+    with pytest.raises(ValueError, match="out of range"):
+        ops.wkv7_decode_layers(wkv, ids[:-1] + [rows], xs)
+    assert torch.equal(wkv, want)

@@ -453,20 +453,31 @@ def _io_table(ptrs: list[list[int]], ys: Sequence[int], offset: int = 0):
     return (ctypes.c_void_p * len(flat))(*flat)
 
 
-def wkv7_decode_layers(wkv: torch.Tensor, ids: torch.Tensor, layer_inputs, *,
+def wkv7_decode_layers(wkv: torch.Tensor, ids, layer_inputs, *,
                        scale: float = 1.0, out_dtype: torch.dtype = torch.bfloat16,
                        row_order: torch.Tensor | None = None) -> list[torch.Tensor]:
     """``wkv7_decode_slots`` of every layer of ``wkv [L, rows, H, 64, 64]`` in
     one launch: ``layer_inputs[l]`` are layer l's ``(r, w, k, v, a, b)``
     ``[B, H, 64]``; ``ids`` and ``row_order`` are device int32 (see
-    ``decode_plan``). Returns the layers' ``y [B, H, 64]``, views of one
+    ``decode_plan``), or ``ids`` are given on the host, then visited in slot
+    order. Host ids of up to 256 rows travel in the kernel arguments (12 layers
+    x 4 slots: 72 us a step with their upload, 57 without). Returns the layers' ``y [B, H, 64]``, views of one
     ``[L, B, H, 64]`` tensor."""
     L, rows, H, stride = check_bank(wkv)
     dev = wkv.device
     if len(layer_inputs) != L:
         raise ValueError(f"expected inputs for {L} layers, got {len(layer_inputs)}")
-    ids = device_ids(ids, rows, dev, "slot_ids")
-    B = int(ids.shape[0])
+    host = None
+    if row_order is None and not (isinstance(ids, torch.Tensor) and ids.is_cuda):
+        host = host_ids(ids, rows, "slot_ids", distinct=True)
+        B = len(host)
+        # (host ids under graph capture are refused by the upload)
+        if B > _lib.WKV7_DECODE_MAX_HOST_IDS or torch.cuda.is_current_stream_capturing():
+            ids, row_order = decode_plan(host, rows, dev, wait=False)
+            host = None
+    else:
+        ids = device_ids(ids, rows, dev, "slot_ids")
+        B = int(ids.shape[0])
     if row_order is not None and not (isinstance(row_order, torch.Tensor) and row_order.is_cuda
                                       and row_order.dtype == torch.int32
                                       and row_order.shape == ids.shape):
@@ -477,9 +488,12 @@ def wkv7_decode_layers(wkv: torch.Tensor, ids: torch.Tensor, layer_inputs, *,
     if B:
         base, step = y.data_ptr(), B * H * HEAD_SIZE * y.element_size()
         io = _io_table(ptrs, [base + l * step for l in range(L)])
-        rc = _lib.load().wkv7_decode_layers(wkv.data_ptr(), stride, L, rows, H, ids.data_ptr(),
-                                            _ptr(row_order), B, io, code, float(scale),
-                                            _stream_ptr(dev))
+        lib, pool, tail = _lib.load(), (wkv.data_ptr(), stride, L, rows, H), (
+            B, io, code, float(scale), _stream_ptr(dev))
+        if host is not None:
+            rc = lib.wkv7_decode_layers_ids(*pool, (ctypes.c_int32 * B)(*host), *tail)
+        else:
+            rc = lib.wkv7_decode_layers(*pool, ids.data_ptr(), _ptr(row_order), *tail)
         _lib.check(rc, "wkv7_decode_layers")
     return list(y.unbind(0))
 

@@ -109,10 +109,8 @@ class WKV7Runner:
         self._check_layers(layer_inputs)
         if any(int(x.shape[0]) != len(slot_batch) for xs in layer_inputs for x in xs):
             raise ValueError("slot_batch and last_tokens length mismatch")
-        ids, order = ops.decode_plan(ops.ids_list(slot_batch, "wkv"), self.bank.num_slots + 1,
-                                     self.device, wait=False)
-        return ops.wkv7_decode_layers(self.bank.wkv, ids, layer_inputs, out_dtype=out_dtype,
-                                      row_order=order)
+        return ops.wkv7_decode_layers(self.bank.wkv, ops.ids_list(slot_batch, "wkv"),
+                                      layer_inputs, out_dtype=out_dtype)
 
     @torch.inference_mode()
     def mixed_step(self, decode_batch: list[dict[str, int]],
