@@ -88,3 +88,16 @@ def test_graph_rejects_wrong_batch(dev):
         dg.set_slots([1, 1, 2])
     with pytest.raises(ValueError):
         dg.set_slots([1, 2, graphed.num_slots + 1])
+
+
+def test_set_slots_is_refused_under_capture(dev):
+    layout = RWKV7StateLayout(n_layer=1, hidden_size=64, num_heads=1, head_dim=64,
+                              head_v_dim=64, dtype=torch.bfloat16)
+    graph = DecodeGraph(RWKV7StateBank(layout, num_slots=4, device=dev), 2)
+    graph.set_slots([1, 3])
+    plan = graph.plan.clone()
+    with torch.cuda.graph(torch.cuda.CUDAGraph()):
+        with pytest.raises(RuntimeError, match="capture"):
+            graph.set_slots([2, 4])
+        plan + 1  # (a graph of one node)
+    assert torch.equal(graph.plan, plan)

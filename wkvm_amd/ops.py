@@ -101,7 +101,10 @@ def upload_ints(values: list[int], device: torch.device, wait: bool = True) -> t
 def refresh_ints(dst: torch.Tensor, values: list[int], event: torch.cuda.Event) -> None:
     """Host integers into a device int32 tensor that a graph reads, ordered on
     the current stream without waiting for it; ``event`` is recorded behind
-    the copy, for a replay on another stream to wait for."""
+    the copy, for a replay on another stream to wait for. Refused under graph
+    capture: a replay would read pinned memory that holds other values by then."""
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("set_slots under graph capture: its ids are host values")
     dst.copy_(torch.tensor(values, dtype=torch.int32, pin_memory=True), non_blocking=True)
     event.record(torch.cuda.current_stream(dst.device))
 
@@ -461,8 +464,8 @@ def wkv7_decode_layers(wkv: torch.Tensor, ids, layer_inputs, *,
     ``[B, H, 64]``; ``ids`` and ``row_order`` are device int32 (see
     ``decode_plan``), or ``ids`` are given on the host, then visited in slot
     order. Host ids of up to 256 rows travel in the kernel arguments (12 layers
-    x 4 slots: 72 us a step with their upload, 57 without). Returns the layers' ``y [B, H, 64]``, views of one
-    ``[L, B, H, 64]`` tensor."""
+    x 4 slots: 72 us a step with their upload, 57 without). Returns the
+    layers' ``y [B, H, 64]``, views of one ``[L, B, H, 64]`` tensor."""
     L, rows, H, stride = check_bank(wkv)
     dev = wkv.device
     if len(layer_inputs) != L:
