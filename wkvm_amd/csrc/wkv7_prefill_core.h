@@ -38,7 +38,7 @@
 // What bounds it: with every compute unit busy the power limit (8 x 4096
 // tokens x 32 heads: 203 us and 2.41 GHz for a launch by itself, 231 us at
 // about 2.1 GHz in a row of them), then the products' and the vector units'
-// work, no longer LDS or issue slots alone: 93 M instructions, 57 M LDS cycles
+// work, no longer LDS or issue slots alone: 95 M instructions, 57 M LDS cycles
 // and 10.5 M bank-conflict cycles per such launch, where one wave per role and
 // SIMD (16 waves, every wave's operands read at the start of its tick, each
 // split by an unpack and a subtraction) took 124 M, 77 M and 21 M, 219 us by

@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kCopyThreads) void slot_zero_kernel(RowMap m, int64
 // A fork of slots within up to kForkFamilies tensors in one launch, its ids in
 // the kernel arguments: id uploads (one per list, each ordered before the copy)
 // and a second family's launch cost 24 of 181 us when 32 slots x 24 layers of the
-// 1.5B shape fork (157 us now, 5.2 TB/s), and nearly all of it for one slot.
+// 1.5B shape fork (157 us now, 5.2 TB/s).
 // Tiles as above; a workgroup's family, pair and row are uniform.
 constexpr int kForkFamilies = 2;
 constexpr int kForkPairs = 128;  // 2 KiB of the 4 KiB of arguments
