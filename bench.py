@@ -590,7 +590,7 @@ def bench_mixed(torch, dev, args, launcher):
     """Config 4: 1.5B, 1024-slot pool; 64 rows prefill U[1, 2048] tokens from
     zero state plus 448 rows decode one token; one decode launch and one varlen
     prefill launch per layer, 24 layers = one scheduler step. Timed with the
-    decode launches on a side stream (the runner's schedule) and on one stream."""
+    decode launches on a side stream and on one, a launch per layer either way."""
     from wkvm_amd import ops, synthetic
 
     L, H, S, NP, ND = 24, 32, 1024, 64, 448
