@@ -4,6 +4,8 @@ rejection, Python validation, and that nothing silently falls back to CPU."""
 from __future__ import annotations
 
 import ctypes
+import gc
+import weakref
 
 import numpy as np
 import pytest
@@ -224,6 +226,39 @@ def test_host_cu_validation():
     for bad in ([1, 7], [0, 5], [0, 4, 3, 7], []):
         with pytest.raises(ValueError):
             ops._host_cu(bad, 7)
+
+
+def test_fla_op_holds_its_plan_across_the_launch(monkeypatch):
+    """The device plan stays alive until the launch call has returned, also when
+    other threads' calls push it out of the cache in between."""
+    plans, held = [], []
+
+    class Lib:
+        @staticmethod
+        def wkv7_prefill_into(*args):
+            ops._PLANS.clear()  # what 256 insertions by other threads do
+            gc.collect()
+            held.append(plans[0]() is not None)
+            return 0
+
+    real_plan = ops._device_plan
+
+    def device_plan(lst, dev):
+        plan = real_plan(lst, dev)
+        plans.append(weakref.ref(plan))
+        return plan
+
+    monkeypatch.setattr(ops, "_device_plan", device_plan)
+    monkeypatch.setattr(ops, "_PLANS", type(ops._PLANS)())
+    monkeypatch.setattr(ops, "_require_cuda", lambda *a: None)
+    monkeypatch.setattr(ops, "_stream_ptr", lambda dev: 0)
+    monkeypatch.setattr(ops, "auto_segments", lambda *a: 1)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(_lib, "load", Lib)
+    xs = [torch.zeros((1, 5, 2, 64), dtype=torch.bfloat16) for _ in range(6)]
+    assert all(x.data_ptr() % 16 == 0 for x in xs)
+    ops.chunk_rwkv7(*xs, cu_seqlens=[0, 2, 5])
+    assert held == [True]
 
 
 def test_longest_first_order():

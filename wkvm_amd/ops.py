@@ -1305,8 +1305,11 @@ def _seq_op(r, w, k, v, a, b, scale, initial_state, output_final_state, cu_seqle
             rc = lib.wkv7_decode_into(*states, None, nseq, *ptrs, *tail)
             _lib.check(rc, "wkv7_decode_into")
         else:
-            plan = _device_plan(host_cu, dev).data_ptr()
-            rc = lib.wkv7_prefill_into(*states, plan, plan + 4 * (nseq + 1), nseq, host_cu[-1],
+            # held until the launch is enqueued: the cache's own reference can go with
+            # another thread's insertions
+            plan = _device_plan(host_cu, dev)
+            cu = plan.data_ptr()
+            rc = lib.wkv7_prefill_into(*states, cu, cu + 4 * (nseq + 1), nseq, host_cu[-1],
                                        *ptrs, *tail)
             _lib.check(rc, "wkv7_prefill_into")
         return y, final
