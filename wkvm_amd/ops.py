@@ -1292,7 +1292,7 @@ def _seq_op(r, w, k, v, a, b, scale, initial_state, output_final_state, cu_seqle
     state = _fla_state(initial_state, nseq, H, dev)
     lens = [host_cu[i + 1] - host_cu[i] for i in range(nseq)]
     decode = nseq > 0 and max(lens) == 1 == min(lens)  # one token per sequence
-    if ptrs and nseq and (decode or auto_segments(H, lens, dev) == 1) and r.dtype == torch.bfloat16:
+    if ptrs and nseq and (decode or auto_segments(H, lens, dev) == 1):
         # every argument is checked: straight to the launch
         lib = _lib.load()
         final = (torch.empty((nseq, H, K, K), dtype=torch.float32, device=dev)
