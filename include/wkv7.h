@@ -290,8 +290,8 @@ int wkv7_segment_chain(float *wkv_layer, int64_t num_rows, int32_t H, const floa
 
 /*
  * The output of a segmented prefill: for every token block,
- * y = y0 + q hin[seg] (seg >= 0) or y = y0 (seg < 0), per head, written in
- * y_dtype.
+ * y = y0 + q hin[seg] (seg >= 0) or y = y0 (seg < 0), per head, in fp32
+ * (operands, products and sums), written in y_dtype.
  *   y0, q    [total_tokens, H, 64] fp32 (the runs' y and y_alt)
  *   blk_tab  [nblk][3] int32 (device): first token, count (<= 64), segment
  */

@@ -9,6 +9,8 @@ compared with the unrounded value."""
 
 from __future__ import annotations
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -800,9 +802,8 @@ def test_segment_chain_and_correct_against_float64(dev, y_dtype):
     """The two combination kernels of the segmented prefill on random
     matrices: H_out = H0 + Phi H_in over 0, 1 and 3 segments, and y = y0 + q
     H_in for token blocks around the 16 tokens of a wave (and one without a
-    correction). The products take q and H_in as bf16 hi + lo parts, each
-    within 2^-18 of its value, without the lo x lo term (2^-18): 2^-16.4 of
-    the summed magnitudes, plus fp32 accumulation of 64 terms."""
+    correction). Both are fp32: 64 products and 64 sums onto the first term,
+    each rounded once, 2^-24 of the summed magnitudes at a time."""
     from wkvm_amd import _lib
 
     lib, H, N = _lib.load(), 3, 64
@@ -847,7 +848,59 @@ def test_segment_chain_and_correct_against_float64(dev, y_dtype):
             t = slice(blk[3 * i], blk[3 * i] + c)
             exact[t] += torch.einsum("thk,hkv->thv", q[t].double(), hin[s].double())
             size[t] += torch.einsum("thk,hkv->thv", q[t].abs().double(), hin[s].abs().double())
-    bar = size * (2.0**-16.4 + 64 * 2.0**-24)
+    bar = size * (66 * 2.0**-24)
     if y_dtype == torch.bfloat16:
         bar = bar + exact.abs() * 2.0**-8
     assert ((y.double() - exact).abs() <= bar).all()
+
+
+@pytest.mark.parametrize("value", [math.nan, math.inf, -math.inf])
+def test_segment_correct_keeps_value_columns_apart(dev, value):
+    """A non-finite entry of H_in reaches its own value column of y alone, as
+    the fp32 sum gives it there; the other 63 columns keep the bits of the
+    finite run."""
+    from wkvm_amd import _lib
+
+    lib, H, N, T, col = _lib.load(), 2, 64, 80, 37
+    g = synthetic.make_generator(67, dev)
+    y0, q, hin = (torch.randn(s, generator=g, device=dev) for s in
+                  ((T, H, N), (T, H, N), (1, H, N, N)))
+    blk = torch.tensor([0, 64, 0, 64, T - 64, 0], dtype=torch.int32, device=dev)
+
+    def run(hin):
+        y = torch.empty((T, H, N), dtype=torch.float32, device=dev)
+        rc = lib.wkv7_segment_correct(T, H, y0.data_ptr(), q.data_ptr(), blk.data_ptr(), 2,
+                                      hin.data_ptr(), 1, y.data_ptr(), _lib.WKV7_Y_F32,
+                                      torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        torch.cuda.synchronize()
+        return y
+
+    want = run(hin)
+    hin[0, 1, 20, col] = value
+    got = run(hin)
+    hit = torch.zeros((H, N), dtype=torch.bool, device=dev)
+    hit[1, col] = True
+    assert torch.equal(got[:, ~hit], want[:, ~hit])
+    exact = y0[:, 1, col] + (q[:, 1] * hin[0, 1, :, col]).sum(-1)
+    assert torch.equal(got[:, 1, col].nan_to_num(7.0), exact.nan_to_num(7.0))
+
+
+def test_segmented_prefill_keeps_value_columns_apart(dev):
+    """The same through the whole segmented prefill: one value column of a
+    state is NaN, the other columns of y and of the final states keep their bits."""
+    H, T, col = 2, 200, 12
+    gen = synthetic.make_generator(69)
+    xs = [synthetic.wkv7_vectors((T, H, 64), gen)[n].to(dev) for n in "rwkvab"]
+    h0 = synthetic.initial_states((1, H, 64, 64), gen).to(dev)
+    got = []
+    for fill in (0.5, math.nan):
+        pool = h0.clone()
+        pool[0, :, :, col] = fill
+        y = ops.wkv7_prefill_segments(pool, [0], [0, T], *xs, segments=4, out_dtype=torch.float32)
+        torch.cuda.synchronize()
+        got.append((y, pool))
+    rest = [c for c in range(64) if c != col]
+    assert torch.equal(got[0][0][..., rest], got[1][0][..., rest])
+    assert torch.equal(got[0][1][..., rest], got[1][1][..., rest])
+    assert got[1][0][..., col].isnan().all()

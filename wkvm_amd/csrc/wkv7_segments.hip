@@ -8,7 +8,7 @@
 // entering segment g:
 //   H_out = H0_g + Phi_g H_in          (wkv7_segment_chain, in segment order)
 //   y_g   = y0_g + q_g H_in            (wkv7_segment_correct, all tokens at once)
-// Both accumulate in fp32; state matrices use the pool layout [j][i] (key j, value i),
+// Both in fp32; state matrices use the pool layout [j][i] (key j, value i),
 // on which Phi acts from the left.
 #include "wkv7_mfma.h"
 
@@ -67,17 +67,24 @@ __global__ __launch_bounds__(kCombThreads) void segment_chain_kernel(
 }
 
 // One block of at most 64 tokens of one head per workgroup, 16 tokens per
-// wave: y^T = y0^T + H_in^T q^T on the matrix cores, H_in and q as bf16 hi + lo
-// (three products per term, ~2^-16 relative) on the fp32 y0 as the accumulator.
-// It moves 564 bytes per token-head and runs near that (16384 tokens x 32
-// heads); as 64 fp32 multiply-adds per value out of LDS it read 16 KiB of LDS
-// per token and took 88 us.
+// wave: y^T = y0^T + H_in^T q^T on the matrix cores, in fp32 throughout (fp32
+// operands and accumulators, y0 as the first term), so that a value column's y
+// depends on that column of H_in alone and rounds as fp32 multiply-adds do.
+// v_mfma_f32_16x16x4_f32, lane l, li = l % 16, lg = l / 16: A lane holds A[li][lg],
+// B lane holds B[lg][li], the accumulator D[4lg .. 4lg+3][li]. k label lg of a
+// step is key 32 kb + 8 lg + e, so that q goes from memory straight to the B
+// operand and H_in comes from LDS in rows of kHinPitch floats: the four rows
+// of a read lie 8 apart, 16 banks from each other. It moves 564 bytes per
+// token-head and runs near that: 16384 tokens x 32 heads 67 us (4.4 TB/s); as
+// scalar multiply-adds out of LDS 88 us, as three bf16 products of hi + lo
+// parts 65 us, at 2^-16 and with a column's non-finite value in its neighbour.
+constexpr int kHinPitch = kHead + 2;
 template <bool kF32Out>
 __global__ __launch_bounds__(kCombThreads) void segment_correct_kernel(
     int64_t total_tokens, int H, const float* __restrict__ y0, const float* __restrict__ q,
     const int32_t* __restrict__ blk_tab, int nblk, const float* __restrict__ hin, int nsegs,
     void* __restrict__ y) {
-  __shared__ __align__(16) uint16_t hs[2][kHead * kPR];  // H_in hi, lo: [key][value column]
+  __shared__ __align__(16) float hs[kHead * kHinPitch];  // H_in: [key][value column]
   const int64_t blk = blockIdx.x / H;
   const int64_t head = blockIdx.x - blk * H;
   if (blk >= nblk) return;
@@ -106,38 +113,27 @@ __global__ __launch_bounds__(kCombThreads) void segment_correct_kernel(
     }
   }
   if (corr) {  // uniform
-    const Neg n = neg_consts();
     const f32x4* src = reinterpret_cast<const f32x4*>(hin + (int64_t(seg) * H + head) * kMat);
 #pragma unroll
     for (int i = 0; i < kMat / 4 / kCombThreads; ++i) {
       const int at = kCombThreads * i + threadIdx.x;
-      uint2 hi, lo;
-      pack_split(src[at], hi, lo, n);
-      const int off = rk_off(at >> 4, 4 * (at & 15));
-      *reinterpret_cast<uint2*>(&hs[0][off]) = hi;
-      *reinterpret_cast<uint2*>(&hs[1][off]) = lo;
-    }
-    uint4 qh[2], ql[2];
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      uint2 h0, l0, h1, l1;
-      pack_split(qv[kb][0], h0, l0, n);
-      pack_split(qv[kb][1], h1, l1, n);
-      qh[kb] = make_uint4(h0.x, h0.y, h1.x, h1.y);
-      ql[kb] = make_uint4(l0.x, l0.y, l1.x, l1.y);
+      const f32x4 h = src[at];
+      float* row = &hs[(at >> 4) * kHinPitch + 4 * (at & 15)];  // 8-byte aligned
+      *reinterpret_cast<float2*>(row) = make_float2(h[0], h[1]);
+      *reinterpret_cast<float2*>(row + 2) = make_float2(h[2], h[3]);
     }
     __syncthreads();
-    // A operand H_in^T: value column 16 ct + li at keys 32 kb + 8 lg .. + 7
-    auto tile = [&](const uint16_t* m, int ct, int kb) {
-      const int r = 32 * kb + 8 * lg + (li >> 2), c = 16 * ct + 4 * (li & 3);
-      const uint2 a = ld_tr(m + rk_off(r, c)), b = ld_tr(m + rk_off(r + 4, c));
-      return make_uint4(a.x, a.y, b.x, b.y);
-    };
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-        acc[ct] = mma32x3(tile(hs[0], ct, kb), tile(hs[1], ct, kb), qh[kb], ql[kb], acc[ct]);
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int ct = 0; ct < 4; ++ct)
+          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              hs[(32 * kb + 8 * lg + e) * kHinPitch + 16 * ct + li], qv[kb][e >> 2][e & 3],
+              acc[ct], 0, 0, 0);
+    // past the last product's 8 passes before a vector instruction reads it
+    asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
   }
   if (!mine) return;
 #pragma unroll

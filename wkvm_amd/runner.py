@@ -42,7 +42,8 @@ class WKV7Runner:
         ``SEGMENT_MIN_TOKENS`` tokens into that many segments that run side by
         side (``ops.wkv7_prefill_segments``); ``"auto"`` picks the count from
         the compute units one chunk leaves idle (``ops.auto_segments``);
-        ``None`` runs every chunk in one pass. Results agree to fp32 rounding."""
+        ``None`` runs every chunk in one pass. Results agree to the
+        scan's rounding (``ops.wkv7_prefill_segments``)."""
         if prefill_chunk < 1:
             raise ValueError("prefill_chunk must be >= 1")
         if prefill_segments is not None and prefill_segments != "auto" and (
