@@ -74,8 +74,8 @@ __global__ __launch_bounds__(kCombThreads) void segment_chain_kernel(
 // B lane holds B[lg][li], the accumulator D[4lg .. 4lg+3][li]. k label lg of a
 // step is key 32 kb + 8 lg + e, so that q goes from memory straight to the B
 // operand and H_in comes from LDS in rows of kHinPitch floats: the four rows
-// of a read lie 8 apart, 16 banks from each other. It moves 564 bytes per
-// token-head and runs near that: 16384 tokens x 32 heads 67 us (4.4 TB/s); as
+// of a read lie 8 apart, 16 banks from each other. The 564 bytes per token-head
+// bound it: 16384 tokens x 32 heads 67 us (4.4 TB/s); as
 // scalar multiply-adds out of LDS 88 us, as three bf16 products of hi + lo
 // parts 65 us, at 2^-16 and with a column's non-finite value in its neighbour.
 constexpr int kHinPitch = kHead + 2;
