@@ -101,3 +101,53 @@ def test_set_slots_is_refused_under_capture(dev):
             graph.set_slots([2, 4])
         plan + 1  # (a graph of one node)
     assert torch.equal(graph.plan, plan)
+
+
+def _busy(dev, stream):
+    """Some milliseconds of work on ``stream``."""
+    with torch.cuda.stream(stream):
+        x = torch.ones((4096, 4096), device=dev)
+        for _ in range(20):
+            x = x @ x * 2.0**-12
+
+
+def test_slots_and_replays_on_different_streams(dev):
+    """set_slots on one stream and replay on another run in the order of the
+    calls, whichever of the streams still has work queued before its part: a
+    replay reads the ids set last, a new set of ids waits for the replay that
+    reads the old ones, and of two sets the later stays."""
+    _, want, graphed = _banks(dev)
+    dg = DecodeGraph(graphed, 2)
+    ref = DecodeGraph(want, 2)
+    xs = [synthetic.order(synthetic.wkv7_vectors((2, 4, 64), synthetic.make_generator(15, dev)))
+          for _ in range(3)]
+    for g in (dg, ref):
+        g.set_inputs(xs)
+    s1, s2 = torch.cuda.Stream(dev), torch.cuda.Stream(dev)
+    _busy(dev, s1)  # (its first call allocates and loads)
+    torch.cuda.synchronize()
+    sets = [[1, 2], [3, 4], [5, 6], [7, 8]]
+    steps = [  # (stream of set_slots, of replay; which of them is busy first)
+        (s1, s2, s1), (s1, s2, s2), (s2, s1, s1), (s2, s1, s2)]
+    for slots in sets:
+        for set_on, replay_on, busy in steps:
+            _busy(dev, busy)
+            with torch.cuda.stream(set_on):
+                dg.set_slots(slots)
+            with torch.cuda.stream(replay_on):
+                dg.replay()
+    for stale in sets[:2]:  # replaced before any replay reads it
+        _busy(dev, s1)
+        with torch.cuda.stream(s1):
+            dg.set_slots(stale)
+        with torch.cuda.stream(s2):
+            dg.set_slots([9, 10])
+            dg.replay()
+    torch.cuda.synchronize()
+    for slots in sets:
+        for _ in steps:
+            ref.step(slots)
+    for _ in sets[:2]:
+        ref.step([9, 10])
+    torch.cuda.synchronize()
+    assert torch.equal(graphed.wkv, want.wkv)

@@ -38,7 +38,7 @@ class DecodeGraph:
         self.bank, self.batch_size = bank, batch_size
         # slot ids in [0, B), visiting order in [B, 2B); the pad row 0 until set
         self.plan = torch.zeros(2 * batch_size, dtype=torch.int32, device=dev)
-        self._slots_set = torch.cuda.Event()
+        self._order = ops.ReplayOrder()
         self.plan[batch_size:] = torch.arange(batch_size, dtype=torch.int32, device=dev)
         # inputs[l] = (r, w, k, v, a, b), each [B, H, 64] bf16 (w = log-decay)
         self.inputs = torch.zeros((L, 6, batch_size, H, HEAD_SIZE), dtype=torch.bfloat16,
@@ -65,7 +65,8 @@ class DecodeGraph:
 
     def set_slots(self, slot_batch) -> None:
         """Validate the batch's slot ids (list of arena slot dicts or ints) and
-        upload them with their slot-sorted visiting order."""
+        upload them with their slot-sorted visiting order, behind the latest
+        ``replay`` on whichever stream it ran."""
         ids = ops.ids_list(slot_batch, "wkv") if slot_batch and isinstance(slot_batch[0], dict) \
             else list(slot_batch)
         if len(ids) != self.batch_size:
@@ -73,12 +74,11 @@ class DecodeGraph:
                              f"{self.batch_size}")
         lst = ops.host_ids(ids, self.bank.num_slots + 1, "slot_ids", distinct=True)
         order = sorted(range(len(lst)), key=lst.__getitem__)
-        ops.refresh_ints(self.plan, lst + order, self._slots_set)
+        self._order.refresh(self.plan, lst + order)
 
     def replay(self) -> torch.Tensor:
         """Run the captured step; returns the static ``y`` [L, B, H, 64]."""
-        torch.cuda.current_stream(self.bank.device).wait_event(self._slots_set)
-        self.graph.replay()
+        self._order.replay(self.graph, self.bank.device)
         return self.y
 
     def step(self, slot_batch, layer_inputs=None) -> torch.Tensor:

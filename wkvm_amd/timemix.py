@@ -270,7 +270,7 @@ class TimeMixDecodeGraph:
         # [2B, 3B] offsets 0..B
         self.plan = torch.cat([torch.arange(1, B + 1), torch.arange(B),
                                torch.arange(B + 1)]).to(torch.int32).to(dev)
-        self._slots_set = torch.cuda.Event()
+        self._order = ops.ReplayOrder()
         self.x = torch.zeros((len(layers), B, D), dtype=torch.bfloat16, device=dev)
         self.o: list[torch.Tensor] = []
         batch = TokenBatch(self.plan[:B], self.plan[2 * B:], self.plan[B:2 * B], B, B, True)
@@ -301,16 +301,16 @@ class TimeMixDecodeGraph:
 
     def set_slots(self, slot_ids) -> None:
         """Validate the batch's slot ids (ints) and upload them with their
-        slot-sorted visiting order."""
+        slot-sorted visiting order, behind the latest ``replay`` on whichever
+        stream it ran."""
         lst = ops.host_ids(slot_ids, self.bank.num_slots + 1, "slot_ids", distinct=True)
         if len(lst) != self.batch_size:
             raise ValueError(f"batch of {len(lst)} slots for a graph of batch size "
                              f"{self.batch_size}")
         order = sorted(range(len(lst)), key=lst.__getitem__)
-        ops.refresh_ints(self.plan[:2 * self.batch_size], lst + order, self._slots_set)
+        self._order.refresh(self.plan[:2 * self.batch_size], lst + order)
 
     def replay(self) -> list[torch.Tensor]:
         """Run the captured step; returns the static outputs ``o`` (L x [B, D])."""
-        torch.cuda.current_stream(self.bank.device).wait_event(self._slots_set)
-        self.graph.replay()
+        self._order.replay(self.graph, self.bank.device)
         return self.o
