@@ -797,6 +797,27 @@ def test_all_layers_in_one_launch_equal_one_launch_each(dev, L, H, lens, y_dtype
     assert torch.equal(wkv, ref)
 
 
+def test_more_sequences_of_all_layers_than_one_launch_holds(dev):
+    """32 layers x 90 sequences x 2048 heads in workgroups of 768 threads pass
+    the 2^32 work items of a launch; one layer does not. All but the first
+    sequence are empty and have a rejected slot."""
+    L, H, n, T = 32, 2048, 90, 16
+    assert L * H * n * 768 >= 1 << 32 > H * n * 768
+    gen = synthetic.make_generator(83, dev)
+    xs = synthetic.order(synthetic.wkv7_vectors((T, H, 64), gen))
+    h0 = synthetic.initial_states((2, H, 64, 64), gen)
+    wkv = h0.expand(L, *h0.shape).contiguous()
+    ids = torch.tensor([1] + [-1] * (n - 1), dtype=torch.int32, device=dev)
+    cu = torch.tensor([0] + [T] * n, dtype=torch.int32, device=dev)
+    ptrs, keep = ops.layer_vectors([xs] * L, (T, H, 64), wkv.device, "prefill")
+    ys = [torch.empty((T, H, 64), dtype=torch.bfloat16, device=dev) for _ in range(L)]
+    ops.wkv7_prefill_layers(wkv, ids, cu, ptrs, ys, 0, T)
+    want = ops.wkv7_prefill_varlen(h0, [1], [0, T], *xs)
+    torch.cuda.synchronize()
+    for layer in range(L):
+        assert torch.equal(ys[layer], want) and torch.equal(wkv[layer], h0)
+
+
 @pytest.mark.parametrize("y_dtype", [torch.bfloat16, torch.float32])
 def test_segment_chain_and_correct_against_float64(dev, y_dtype):
     """The two combination kernels of the segmented prefill on random

@@ -114,8 +114,12 @@ extern "C" int wkv7_prefill_layers(float* wkv, int64_t layer_stride, int32_t lay
       return WKV7_ERR_SHAPE;
   }
   const Runs runs{nullptr, nullptr, nseq, nullptr, 0, nullptr, nullptr, nullptr, 0};
-  for (int32_t l = 0; l < layers; l += kMaxLayers) {
-    const int32_t n = layers - l < kMaxLayers ? layers - l : kMaxLayers;
+  // as many layers per launch as its argument table holds and its work items
+  // fit into 32 bits
+  const int64_t fit = int64_t(UINT32_MAX) / (int64_t(nseq) * H * kWaves * kWave);
+  const int32_t step = fit < 1 ? 1 : fit < kMaxLayers ? int32_t(fit) : kMaxLayers;
+  for (int32_t l = 0; l < layers; l += step) {
+    const int32_t n = layers - l < step ? layers - l : step;
     PrefillArgs p{wkv + l * layer_stride, num_rows,     H,         slot_ids, cu_seqlens, seq_order,
                   nseq,                   total_tokens, zero_init, scale,    runs};
     p.layer_stride = layer_stride;
