@@ -632,6 +632,27 @@ def test_runner_segmented_prefill_matches_one_pass(dev):
         assert U.rel_l2(U.f64(finals[i]), U.f64(finals[0])) <= 1e-4
 
 
+@pytest.mark.parametrize("segments", [None, 2])
+def test_runner_prefill_of_longer_vectors(dev, segments):
+    """The prompt is as long as the first layer's r; vectors with more tokens
+    are read up to there."""
+    lay = RWKV7StateLayout(n_layer=2, hidden_size=128, num_heads=2, head_dim=64, head_v_dim=64,
+                           dtype=torch.bfloat16)
+    T, gen = 2100, synthetic.make_generator(73, dev)
+    exact = [synthetic.order(synthetic.wkv7_vectors((T, 2, 64), gen)) for _ in range(2)]
+    pad = lambda x: torch.cat([x, x[:7]])  # noqa: E731
+    longer = [[exact[0][0]] + [pad(x) for x in exact[0][1:]], [pad(x) for x in exact[1]]]
+    got = []
+    for inputs in (exact, longer):
+        bank = RWKV7StateBank(lay, num_slots=1, device=dev)
+        run = WKV7Runner(bank, prefill_chunk=2048, prefill_segments=segments)
+        got.append((torch.stack(run.prefill(inputs, {"wkv": 1, "shift": 1})), bank.wkv))
+    torch.cuda.synchronize()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    with pytest.raises(ValueError, match="prefill"):
+        run.prefill([exact[0], [x[:-1] for x in exact[1]]], {"wkv": 1, "shift": 1})
+
+
 def test_fla_signature_long_single_sequence_runs_segmented(dev):
     """chunk_rwkv7 with one long sequence picks the segmented form (few busy
     compute units) and still matches the oracle, from an initial state and

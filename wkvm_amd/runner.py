@@ -76,7 +76,11 @@ class WKV7Runner:
         # device plans (offsets 0, n and the one-sequence order), uploaded once
         # per chunk length rather than once per layer
         plans: dict[int, torch.Tensor] = {}
-        ptrs, keep = ops.layer_vectors(layer_inputs, (T, H, 64), self.bank.wkv.device, "prefill")
+        # the first layer's r says how many tokens there are, longer vectors are
+        # read up to there
+        layer_inputs = [xs if all(x.shape[0] == T for x in xs) else [x[:T] for x in xs]
+                        for xs in layer_inputs]
+        ptrs = None
         for start in range(0, T, self.prefill_chunk):
             n = min(self.prefill_chunk, T - start)
             if n not in plans:
@@ -89,6 +93,9 @@ class WKV7Runner:
                                               *[x[start:start + n] for x in xs], segments=G,
                                               out=ys[layer][start:start + n])
             else:
+                if ptrs is None:
+                    ptrs, keep = ops.layer_vectors(layer_inputs, (T, H, 64),
+                                                   self.bank.wkv.device, "prefill")
                 ops.wkv7_prefill_layers(self.bank.wkv, ids, plan[:2], ptrs, ys, start, n,
                                         seq_order=plan[2:])
         return ys
