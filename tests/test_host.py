@@ -306,6 +306,26 @@ def test_runner_argument_errors():
 
 # -- synthetic inputs ---------------------------------------------------------------------------
 
+@pytest.mark.parametrize("layers,tokens,count,want", [
+    (1, 2048, 4, 4), (1, 2047, 4, 1), (2, 4096, 4, 4), (2, 4095, 4, 1), (3, 16384, 4, 1),
+    (3, 16384, 8, 8), (4, 16384, 8, 8), (5, 65536, 8, 1), (24, 65536, 8, 1)])
+def test_runner_auto_segments_only_for_few_layers(monkeypatch, layers, tokens, count, want):
+    """A launch over all layers fills the units that one layer's chunk leaves
+    idle: from a few layers on "auto" runs every chunk in one pass."""
+    class FakeLayout:
+        n_layer = layers
+
+    class FakeBank:
+        layout = FakeLayout()
+        num_slots = 4
+        device = torch.device("cpu")
+
+    monkeypatch.setattr(ops, "auto_segments", lambda H, lens, device: count)
+    assert WKV7Runner(FakeBank(), prefill_segments="auto")._segments(tokens, 32) == want
+    if tokens >= 2048:
+        assert WKV7Runner(FakeBank(), prefill_segments=3)._segments(tokens, 32) == 3
+
+
 def test_synthetic_distributions_and_determinism():
     g1, g2 = synthetic.make_generator(7), synthetic.make_generator(7)
     a1 = synthetic.wkv7_vectors((32, 4, 64), g1)

@@ -32,16 +32,17 @@ LayerInputs = Sequence[torch.Tensor]  # (r, w, k, v, a, b)
 
 
 class WKV7Runner:
-    # Chunks at least this long run segmented when ``prefill_segments`` is set
-    # (the segmented form is faster from about 2k tokens of one sequence).
+    # Chunks at least this long run segmented when ``prefill_segments`` is a
+    # count (one layer's segments are faster from about 2k tokens on).
     SEGMENT_MIN_TOKENS = 2048
 
     def __init__(self, bank: RWKV7StateBank, prefill_chunk: int = 512,
                  prefill_segments: int | str | None = None) -> None:
         """``prefill_segments``: cut each prefill chunk of at least
         ``SEGMENT_MIN_TOKENS`` tokens into that many segments that run side by
-        side (``ops.wkv7_prefill_segments``); ``"auto"`` picks the count from
-        the compute units one chunk leaves idle (``ops.auto_segments``);
+        side (``ops.wkv7_prefill_segments``), a layer at a time; ``"auto"``
+        picks the count from the compute units one layer's chunk leaves idle
+        (``ops.auto_segments``), for banks of so few layers that it pays;
         ``None`` runs every chunk in one pass. Results agree to the
         scan's rounding (``ops.wkv7_prefill_segments``)."""
         if prefill_chunk < 1:
@@ -104,7 +105,15 @@ class WKV7Runner:
         if self.prefill_segments is None or n < self.SEGMENT_MIN_TOKENS:
             return 1
         if self.prefill_segments == "auto":
-            return ops.auto_segments(H, [n], self.device)
+            G = ops.auto_segments(H, [n], self.device)
+            L = self.bank.layout.n_layer
+            # One launch runs all layers side by side, the segmented form one
+            # after the other, each with about twice the arithmetic and 70 us of
+            # launches and upload. us, segmented against one launch: 16,384 tokens
+            # x 12 heads in 8 segments, 3 layers 462 / 542, 12 layers 1839 / 743;
+            # x 32 heads in 4, 2 layers 598 / 724, 3 layers 832 / 684; 4,096 tokens
+            # x 32 heads in 4, 1 layer 106 / 150, 2 layers 195 / 198.
+            return G if L == 1 or (2 * L <= G and n >= 512 * L * G) else 1
         return self.prefill_segments
 
     @torch.inference_mode()
