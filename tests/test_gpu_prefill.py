@@ -775,6 +775,34 @@ def test_half_and_quarter_heads_bit_identical_to_whole_heads(dev, y_dtype):
     _check(pool.numpy(), ids, np.array(cu), U.vec_bits(vecs), got[0][1], got[0][0], False)
 
 
+@pytest.mark.parametrize("H", [2, 72, 200])
+def test_no_row_past_the_end_counts(dev, H):
+    """Sequences of one to nine sub-chunks, whole and with a remainder, with
+    NaN in every row before and behind them, against the oracle: in quarter,
+    half and whole heads."""
+    lens = [16 * n - cut for n in range(1, 10) for cut in (0, 5, 15)]
+    gen = synthetic.make_generator(89)
+    pool = synthetic.initial_states((1, H, 64, 64), gen)
+    vecs = synthetic.wkv7_vectors((144, H, 64), gen)
+    bits = U.vec_bits(vecs)
+    ids = torch.zeros(1, dtype=torch.int32, device=dev)
+    for n in lens:
+        xs = []
+        for name in "rwkvab":
+            x = torch.full((n + 160, H, 64), math.nan, dtype=torch.bfloat16, device=dev)
+            x[20:20 + n] = vecs[name][:n].to(dev)
+            xs.append(x)
+        wkv = pool.to(dev)[None]
+        y = torch.full((n + 160, H, 64), 7.0, dtype=torch.float32, device=dev)
+        ptrs, keep = ops.layer_vectors([xs], xs[0].shape, wkv.device, "prefill")
+        cu = torch.tensor([0, n], dtype=torch.int32, device=dev)
+        ops.wkv7_prefill_layers(wkv, ids, cu, ptrs, [y], 20, n)
+        torch.cuda.synchronize()
+        assert (y[:20] == 7).all() and (y[20 + n:] == 7).all()
+        _check(pool.numpy(), [0], np.array([0, n]), [b[:n] for b in bits], wkv[0], y[20:20 + n],
+               False)
+
+
 def test_inputs_past_one_gib_of_a_sequence(dev):
     """A sequence whose inputs pass the 1 GiB at which the row loads move
     their base forward gives the same bits as its two halves run one after

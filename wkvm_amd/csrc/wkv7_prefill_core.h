@@ -45,8 +45,9 @@
 // itself and 254 us in a row. With few heads the state wave's dependent chain
 // (about 0.43 us per tick by itself) and the operand waves beside it.
 // A sequence of one sub-chunk is nearly all fill, one tick longer here than in
-// that kernel: 64 x 8 tokens x 32 heads 44.7 us against 39.9, 32 x 40 tokens
-// 31.5 against 32.1, 16 x 512 tokens 67.5 against 75.6.
+// that kernel, so no role works past the sub-chunk after the end: 64 x 8 tokens
+// x 32 heads 40.8 us (44.7 with the pipeline running on over zero rows, 39.8
+// there), 32 x 40 tokens 29.7 (31.5, 32.4).
 //
 // Precision: MFMA operands that are not exact bf16 inputs are split into bf16
 // hi + lo parts, a product formed as hi*hi + hi*lo + lo*hi with fp32
@@ -326,9 +327,10 @@ __device__ __forceinline__ void operand_role(Shared& sm, int64_t n_sub, int lane
   part &= 1;
   end_tick();  // the first rows' fill tick
   if (odd) end_tick();
-  // Sub-chunk j takes ticks j-4 and j-3; the last tick is n_sub - 1. (Sub-chunks
-  // past the end work on zero rows; of them only k and v of the first are read.)
-  for (int64_t j = odd; j < n_sub + 4; j += 2) {
+  // Sub-chunk j takes ticks j-4 and j-3; the last tick is n_sub - 1. (The
+  // sub-chunk past the end, of zero rows, is the last one: its K~ is read.)
+  int64_t j = odd;
+  for (; j <= n_sub; j += 2) {
     Operands<kScaled, kEarlyB> op;
     {
       SubIn d;
@@ -336,11 +338,10 @@ __device__ __forceinline__ void operand_role(Shared& sm, int64_t n_sub, int lane
       op.first(d, lane, n);
     }
     end_tick();
-    if (j < n_sub + 3) {
-      op.second(sm.slot[j & (kRing - 1)], lane, part, scale, n);
-      end_tick();
-    }
+    op.second(sm.slot[j & (kRing - 1)], lane, part, scale, n);
+    end_tick();
   }
+  for (; j < n_sub + 4; ++j) end_tick();
 }
 
 // ---- scores ---------------------------------------------------------------------------
@@ -434,10 +435,11 @@ __device__ __forceinline__ void stage_inverse(Shared& sm, int64_t j, int lane) {
 
 __device__ __forceinline__ void inverse_role(Shared& sm, int64_t n_sub, int lane) {
   for (int i = 0; i < 4; ++i) end_tick();
-  for (int64_t j = 0; j < n_sub + 1; ++j) {
+  for (int64_t j = 0; j < n_sub; ++j) {
     stage_inverse(sm, j, lane);
     end_tick();
   }
+  end_tick();
 }
 
 // ---- io -------------------------------------------------------------------------------
@@ -554,18 +556,21 @@ struct YRows {
 
 // At the end of tick k sub-chunk k+5's rows must have landed (the operand
 // waves read them in the next tick): everything but the two sub-chunks' loads
-// asked for after it.
+// asked for after it. The last sub-chunk asked for is the one past the end.
 __device__ __forceinline__ void io_role(Shared& sm, const Inputs& in, const SeqGeom& g,
                                         int64_t n_sub, int lane, bool kvz) {
   RowSrc src(in, g, lane, kvz);
   src.issue(sm, 0);
   src.issue(sm, 1);
-  for (int64_t j = 2; j < n_sub + 7; ++j) {  // tick j - 7
+  for (int64_t j = 2; j <= n_sub; ++j) {  // tick j - 7
     src.issue(sm, j);
     wait_vm<2 * kLoads>();
     end_tick();
   }
-  wait_vm<0>();  // no load may land in LDS after the workgroup ends
+  wait_vm<kLoads>();
+  end_tick();
+  wait_vm<0>();
+  for (int i = 0; i < 5; ++i) end_tick();
 }
 
 // Pair 1's wave also stores the y rows of the sub-chunk before the state
@@ -576,7 +581,7 @@ __device__ __forceinline__ void score_role(Shared& sm, const SeqGeom& g, int64_t
   const Neg n = neg_consts();
   for (int i = 0; i < 3; ++i) end_tick();
   for (int i = 0; i < 3; ++i) {  // ticks -2 .. 0
-    stage_scores<pair>(sm, i, lane, n);
+    if (i < n_sub) stage_scores<pair>(sm, i, lane, n);
     end_tick();
   }
   YRows<kF32Out, kCols> rows;
@@ -585,7 +590,7 @@ __device__ __forceinline__ void score_role(Shared& sm, const SeqGeom& g, int64_t
       rows.read(sm, k - 1, lane, col0);
       rows.write(y, k - 1, g, lane, col0);
     }
-    stage_scores<pair>(sm, k + 2, lane, n);
+    if (k + 2 < n_sub) stage_scores<pair>(sm, k + 2, lane, n);
     end_tick();
   }
   if constexpr (pair == 1) {
@@ -762,7 +767,8 @@ __device__ __forceinline__ void state_role(Shared& sm, const float* hsrc, float*
       stage_state<kF32Out>(sm, st, in, k, lane, col0, n);
       end_tick();
     }
-    // the sub-chunk past the end has k = v = 0: hk is the final state
+    // the sub-chunk past the end has k = v = 0: hk is the final state (of its
+    // other operands nothing is made, and nothing of what they give is used)
 #pragma unroll
     for (int jb = 0; jb < 4; ++jb) h[jb] = st.hk[jb];
   }
