@@ -38,8 +38,8 @@ int device_cus() {
   return n;
 }
 
-// p: every field but layers and io, which come from io[0 .. layers).
-int prefill_launch(PrefillArgs& p, int32_t layers, const wkv7_layer_io* io, int32_t y_dtype,
+// p: every field but layers.
+int prefill_launch(PrefillPlan& p, int32_t layers, const wkv7_layer_io* io, int32_t y_dtype,
                    void* stream) {
   const int64_t items = int64_t(p.nseq) * p.H * layers, cus = device_cus();
   // A launch that leaves half or more of the compute units idle splits each
@@ -53,11 +53,10 @@ int prefill_launch(PrefillArgs& p, int32_t layers, const wkv7_layer_io* io, int3
   const int64_t blocks = items * split;
   if (blocks > int64_t(0x7fffffff)) return WKV7_ERR_ARG;
   p.layers = layers;
-  for (int32_t l = 0; l < layers; ++l) p.io[l] = io[l];
   hipStream_t s = as_stream(stream);
   const bool f32 = y_dtype == WKV7_Y_F32, scaled = p.scale != 1.0f;
-  if (split > 1) return prefill_split_launch(split, unsigned(blocks), s, f32, scaled, p);
-  return launch_form<WholeHead>(unsigned(blocks), s, f32, scaled, p);
+  if (split > 1) return prefill_split_launch(split, unsigned(blocks), s, f32, scaled, p, io);
+  return launch_form<WholeHead>(unsigned(blocks), s, f32, scaled, p, io);
 }
 
 // y rows are stored as 8-byte (bf16) or 16-byte (fp32) vectors
@@ -89,7 +88,7 @@ extern "C" int wkv7_prefill_varlen(float* wkv_layer, int64_t num_rows, int32_t H
   if (total_tokens > 0 && (!r || !w || !k || !v || !a || !b || !y)) return WKV7_ERR_ARG;
   if (!inputs_aligned(r, w, k, v, a, b) || !y_aligned(y, y_dtype)) return WKV7_ERR_SHAPE;
   const Runs runs{nullptr, nullptr, nseq, nullptr, 0, nullptr, nullptr, nullptr, 0};
-  PrefillArgs p{wkv_layer, num_rows,     H,         slot_ids, cu_seqlens, seq_order,
+  PrefillPlan p{wkv_layer, num_rows,     H,         slot_ids, cu_seqlens, seq_order,
                 nseq,      total_tokens, zero_init, scale,    runs};
   const wkv7_layer_io io{r, w, k, v, a, b, y};
   return prefill_launch(p, 1, &io, y_dtype, stream);
@@ -120,7 +119,7 @@ extern "C" int wkv7_prefill_layers(float* wkv, int64_t layer_stride, int32_t lay
   const int32_t step = fit < 1 ? 1 : fit < kMaxLayers ? int32_t(fit) : kMaxLayers;
   for (int32_t l = 0; l < layers; l += step) {
     const int32_t n = layers - l < step ? layers - l : step;
-    PrefillArgs p{wkv + l * layer_stride, num_rows,     H,         slot_ids, cu_seqlens, seq_order,
+    PrefillPlan p{wkv + l * layer_stride, num_rows,     H,         slot_ids, cu_seqlens, seq_order,
                   nseq,                   total_tokens, zero_init, scale,    runs};
     p.layer_stride = layer_stride;
     const int rc = prefill_launch(p, n, io + l, y_dtype, stream);
@@ -154,7 +153,7 @@ extern "C" int wkv7_prefill_runs(float* wkv_layer, int64_t num_rows, int32_t H,
     return WKV7_ERR_SHAPE;
   const Runs runs{run_flags, cu_alt,   n_primary, state_alt, alt_rows,
                   y_alt ? y_alt : y, state_in, in_ids,    in_rows};
-  PrefillArgs p{wkv_layer, num_rows,     H,         slot_ids, cu_seqlens, seq_order,
+  PrefillPlan p{wkv_layer, num_rows,     H,         slot_ids, cu_seqlens, seq_order,
                 nseq,      total_tokens, zero_init, scale,    runs};
   const wkv7_layer_io io{r, w, k, v, a, b, y};
   return prefill_launch(p, 1, &io, y_dtype, stream);
@@ -178,7 +177,7 @@ extern "C" int wkv7_prefill_into(const float* state_in, int64_t in_rows, const i
   if (!inputs_aligned(r, w, k, v, a, b) || !y_aligned(y, y_dtype)) return WKV7_ERR_SHAPE;
   // no state_in: zero initial state; no state_out: no final state written
   const Runs runs{nullptr, nullptr, nseq, nullptr, 0, nullptr, state_in, in_ids, in_rows};
-  PrefillArgs p{state_out, state_out ? out_rows : 0, H,                out_ids, cu_seqlens, seq_order,
+  PrefillPlan p{state_out, state_out ? out_rows : 0, H,                out_ids, cu_seqlens, seq_order,
                 nseq,      total_tokens,             state_in ? 0 : 1, scale,   runs};
   const wkv7_layer_io io{r, w, k, v, a, b, y};
   return prefill_launch(p, 1, &io, y_dtype, stream);

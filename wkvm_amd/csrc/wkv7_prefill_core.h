@@ -45,9 +45,10 @@
 // itself and 254 us in a row. With few heads the state wave's dependent chain
 // (about 0.43 us per tick by itself) and the operand waves beside it.
 // A sequence of one sub-chunk is nearly all fill, one tick longer here than in
-// that kernel, so no role works past the sub-chunk after the end: 64 x 8 tokens
-// x 32 heads 40.8 us (44.7 with the pipeline running on over zero rows, 39.8
-// there), 32 x 40 tokens 29.7 (31.5, 32.4).
+// that kernel, so no role works past the sub-chunk after the end and a
+// workgroup finds its work in 32-bit arithmetic: 64 x 8 tokens x 32 heads
+// 37.8 us (44.7 with the pipeline running on over zero rows and 64-bit
+// divisions; 39.8 there), 32 x 40 tokens 28.2 (31.5, 32.0).
 //
 // Precision: MFMA operands that are not exact bf16 inputs are split into bf16
 // hi + lo parts, a product formed as hi*hi + hi*lo + lo*hi with fp32
@@ -166,7 +167,7 @@ struct Runs {
 // `layers` layers share the plan: layer l's states are at wkv + l *
 // layer_stride, its vectors io[l] (one launch instead of a layer's launch
 // after the other's tail).
-struct PrefillArgs {
+struct PrefillPlan {
   float* wkv;  // final states, and initial ones unless runs.state_in or zero_init; null: none
   int64_t num_rows;
   int H;
@@ -178,13 +179,19 @@ struct PrefillArgs {
   Runs runs;
   int layers;
   int64_t layer_stride;
-  wkv7_layer_io io[kMaxLayers];
+};
+
+// A launch's arguments: one layer's vectors, or the table of kMaxLayers (1.75
+// KiB, of which a launch of one layer would copy 56 bytes for its own).
+template <int N>
+struct PrefillArgs : PrefillPlan {
+  wkv7_layer_io io[N];
 };
 
 // Launches the forms of wkv7_prefill_split.hip: `split` (2 or 4) workgroups
 // per (sequence, head).
 int prefill_split_launch(int split, unsigned blocks, hipStream_t s, bool f32_out, bool scaled,
-                         const PrefillArgs& p);
+                         const PrefillPlan& p, const wkv7_layer_io* io);
 
 namespace {
 
@@ -804,8 +811,8 @@ enum Role : int { kState, kOperand, kScore, kInverse, kIo, kNone };
 // (wave w runs on SIMD w % 4).
 constexpr int kWaves = 12;
 
-template <class Form, bool kF32Out, bool kScaled>
-__global__ __launch_bounds__(kWaves * kWave) void prefill_kernel(const PrefillArgs p) {
+template <class Form, bool kF32Out, bool kScaled, int N>
+__global__ __launch_bounds__(kWaves * kWave) void prefill_kernel(const PrefillArgs<N> p) {
   constexpr int kCols = Form::kStateWaves * 16;  // value columns per workgroup
   constexpr int kSplit = kHead / kCols;                     // workgroups per (sequence, head)
   __shared__ Shared sm;
@@ -814,13 +821,14 @@ __global__ __launch_bounds__(kWaves * kWave) void prefill_kernel(const PrefillAr
   // wave-uniform by construction; through readfirstlane the compiler knows it,
   // so the role branches are scalar branches
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  const int64_t item = blockIdx.x / kSplit;
-  // sequences outermost: the longest ones of every layer start first
-  const int64_t per_seq = int64_t(p.layers) * p.H;
-  const int64_t pos = item / per_seq;
-  const int64_t layer = (item - pos * per_seq) / p.H;
-  const int64_t head = item - pos * per_seq - layer * p.H;
-  const wkv7_layer_io& io = p.io[layer];
+  // sequences outermost: the longest ones of every layer start first (a
+  // launch's workgroups fit 32 bits)
+  const uint32_t item = blockIdx.x / kSplit, heads = uint32_t(p.H);
+  const uint32_t per_seq = N == 1 ? heads : uint32_t(p.layers) * heads;
+  const uint32_t at = item / per_seq, rest = item - at * per_seq;
+  const uint32_t layer_at = N == 1 ? 0 : rest / heads;
+  const int64_t pos = at, layer = layer_at, head = rest - layer_at * heads;
+  const wkv7_layer_io& io = p.io[layer_at];
   const int64_t seq = p.seq_order ? int64_t(p.seq_order[pos]) : pos;
   if (seq < 0 || seq >= p.nseq) return;  // uniform: the whole block leaves
   const Runs& runs = p.runs;
@@ -881,17 +889,27 @@ __global__ __launch_bounds__(kWaves * kWave) void prefill_kernel(const PrefillAr
   }
 }
 
-template <class Form>
-int launch_form(unsigned blocks, hipStream_t s, bool f32_out, bool scaled, const PrefillArgs& p) {
+template <class Form, int N>
+int launch_layers(unsigned blocks, hipStream_t s, bool f32_out, bool scaled, const PrefillPlan& p,
+                  const wkv7_layer_io* io) {
+  PrefillArgs<N> a{p, {}};
+  for (int l = 0; l < p.layers; ++l) a.io[l] = io[l];
   const dim3 grid(blocks), threads(kWaves * kWave);
   if (f32_out) {
-    if (scaled) prefill_kernel<Form, true, true><<<grid, threads, 0, s>>>(p);
-    else prefill_kernel<Form, true, false><<<grid, threads, 0, s>>>(p);
+    if (scaled) prefill_kernel<Form, true, true, N><<<grid, threads, 0, s>>>(a);
+    else prefill_kernel<Form, true, false, N><<<grid, threads, 0, s>>>(a);
   } else {
-    if (scaled) prefill_kernel<Form, false, true><<<grid, threads, 0, s>>>(p);
-    else prefill_kernel<Form, false, false><<<grid, threads, 0, s>>>(p);
+    if (scaled) prefill_kernel<Form, false, true, N><<<grid, threads, 0, s>>>(a);
+    else prefill_kernel<Form, false, false, N><<<grid, threads, 0, s>>>(a);
   }
   return launch_status();
+}
+
+template <class Form>
+int launch_form(unsigned blocks, hipStream_t s, bool f32_out, bool scaled, const PrefillPlan& p,
+                const wkv7_layer_io* io) {
+  return p.layers == 1 ? launch_layers<Form, 1>(blocks, s, f32_out, scaled, p, io)
+                       : launch_layers<Form, kMaxLayers>(blocks, s, f32_out, scaled, p, io);
 }
 
 }  // namespace

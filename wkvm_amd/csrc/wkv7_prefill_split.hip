@@ -28,9 +28,9 @@ struct QuarterHead {
 }  // namespace
 
 int prefill_split_launch(int split, unsigned blocks, hipStream_t s, bool f32_out, bool scaled,
-                         const PrefillArgs& p) {
-  if (split == 2) return launch_form<HalfHead>(blocks, s, f32_out, scaled, p);
-  return launch_form<QuarterHead>(blocks, s, f32_out, scaled, p);
+                         const PrefillPlan& p, const wkv7_layer_io* io) {
+  if (split == 2) return launch_form<HalfHead>(blocks, s, f32_out, scaled, p, io);
+  return launch_form<QuarterHead>(blocks, s, f32_out, scaled, p, io);
 }
 
 }  // namespace wkv7
