@@ -775,6 +775,26 @@ def test_half_and_quarter_heads_bit_identical_to_whole_heads(dev, y_dtype):
     _check(pool.numpy(), ids, np.array(cu), U.vec_bits(vecs), got[0][1], got[0][0], False)
 
 
+def test_splits_of_long_launches_bit_identical(dev):
+    """Launches of more than 768 tokens per sequence, of 3/4 of the CUs in
+    quarter heads and of all in half heads, and the next larger ones: the same
+    heads give the same bits."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    counts = [cus * 3 // 16, cus * 3 // 16 + 1, cus // 2, cus // 2 + 1]
+    T, gen = 770, synthetic.make_generator(91, dev)
+    vecs = synthetic.order(synthetic.wkv7_vectors((T, counts[-1], 64), gen))
+    pool = synthetic.initial_states((1, counts[-1], 64, 64), gen)
+    got = []
+    for H in counts:
+        g = pool[:, :H].clone()
+        y = ops.wkv7_prefill_varlen(g, [0], [0, T], *[x[:, :H].contiguous() for x in vecs])
+        got.append((y, g))
+    torch.cuda.synchronize()
+    H = counts[0]
+    for y, g in got[1:]:
+        assert torch.equal(y[:, :H], got[0][0]) and torch.equal(g[:, :H], got[0][1])
+
+
 @pytest.mark.parametrize("H", [2, 72, 200])
 def test_no_row_past_the_end_counts(dev, H):
     """Sequences of one to nine sub-chunks, whole and with a remainder, with

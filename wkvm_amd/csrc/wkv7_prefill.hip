@@ -48,8 +48,13 @@ int prefill_launch(PrefillPlan& p, int32_t layers, const wkv7_layer_io* io, int3
   // state waves share the unit, and the preparation is repeated by each
   // workgroup, which costs nothing while a unit stays free for it: 4 x 1500
   // tokens x 32 heads 77.7 us whole, 73.5 in halves, 134.8 in quarters (which
-  // no longer run side by side); 4096 tokens x 32 heads 136 us in quarters.
-  const int split = 4 * items <= cus ? 4 : 2 * items <= cus ? 2 : 1;
+  // no longer run side by side). It costs power, though: where a launch is long
+  // enough to run into the limit, quarters on more than three quarters of the
+  // units are slower than halves on half as many. us for 2000 tokens, halves /
+  // quarters: 48 heads 82 / 78, 56 82 / 85, 64 83 / 87; 64 heads x 512 tokens 25.5 /
+  // 24.9, x 900 40.1 / 42.2.
+  const bool hot = p.total_tokens > 768 * int64_t(p.nseq);
+  const int split = 4 * items <= (hot ? cus * 3 / 4 : cus) ? 4 : 2 * items <= cus ? 2 : 1;
   const int64_t blocks = items * split;
   if (blocks > int64_t(0x7fffffff)) return WKV7_ERR_ARG;
   p.layers = layers;
