@@ -547,7 +547,10 @@ int wkv7_proj_grouped(int64_t m, const wkv7_proj_group *groups, int32_t ngroups,
  * device (0: none). With at least this many bytes (16-byte aligned) it may
  * split long k over several workgroups, whose fp32 partials a second kernel
  * sums in a fixed order; with less it runs unsplit. Both give results within
- * one bf16 ulp of the exact product; each is deterministic. */
+ * one bf16 ulp of the exact product; each is deterministic. Up to
+ * WKV7_PROJ_FEW_ROWS rows the products this would split run in a kernel of their
+ * own that leaves the workspace alone: callers need not bring one. */
+#define WKV7_PROJ_FEW_ROWS 16
 size_t wkv7_proj_workspace_bytes(int64_t m, const wkv7_proj_group *groups, int32_t ngroups);
 
 /*

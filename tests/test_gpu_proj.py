@@ -129,10 +129,10 @@ def test_rejected_arguments(dev):
 
 
 def test_split_k_partials_and_unsplit_fallback(dev):
-    """A long-k product with few rows splits k over several workgroups when
-    given the workspace it asks for (the last part holding the 32-wide k
-    tail), and runs unsplit without one. Both are within one bf16 ulp of the
-    exact product and each repeats bit for bit."""
+    """A long-k product with few rows, with the split-k workspace it asks for
+    and without one (in the kernel of one row tile it needs none; above 16 rows
+    see test_split_k_above_the_row_tile): both are within one bf16 ulp of the
+    exact product and the first repeats bit for bit."""
     from wkvm_amd import _lib
 
     lib = _lib.load()
@@ -162,8 +162,9 @@ def test_split_k_partials_and_unsplit_fallback(dev):
 
 
 def test_split_k_over_several_groups(dev):
-    """Several products with few rows split k together (different n, one
-    with bias and sigmoid); every output within one bf16 ulp."""
+    """Several products with few rows and long k, which ask for a split-k
+    workspace together (different n, one with bias and sigmoid); every output
+    within one bf16 ulp."""
     from wkvm_amd import _lib
 
     gen = torch.Generator().manual_seed(41)
@@ -222,10 +223,48 @@ def test_few_rows(dev, M, ks, ns):
         assert bool((buf[:, y.shape[1]:] == 7.0).all())
 
 
-def test_split_k_above_the_row_tile(dev):
-    """17 rows of long k and few columns: the k split of the tiled kernel."""
+@pytest.mark.parametrize("M", [17, 32])
+@pytest.mark.parametrize("with_workspace", [True, False])
+def test_split_k_above_the_row_tile(dev, M, with_workspace):
+    """More than 16 rows of long k and few columns: the k split of the tiled
+    kernel with the workspace it asks for (each repeat the same bits), and the
+    unsplit form without."""
+    from wkvm_amd import _lib
+
+    lib = _lib.load()
     gen = torch.Generator().manual_seed(71)
-    x, w = _rand((17, 2080), gen, dev), _rand((1000, 2080), gen, dev, 1 / math.sqrt(2080))
-    b = _rand((1000,), gen, dev)
+    K, N = 2080, 1000
+    x, w = _rand((M, K), gen, dev), _rand((N, K), gen, dev, 1 / math.sqrt(K))
+    b = _rand((N,), gen, dev)
+    arr, outs = (_lib.ProjGroup * 1)(), []
+    for _ in range(2):
+        y = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+        arr[0] = _lib.ProjGroup(x.data_ptr(), w.data_ptr(), b.data_ptr(), y.data_ptr(), K, K, N,
+                                N, K, _lib.WKV7_ACT_TANH, 0)
+        ws_bytes = int(lib.wkv7_proj_workspace_bytes(M, arr, 1))
+        assert ws_bytes > 0
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        rc = lib.wkv7_proj_grouped(M, arr, 1, ws.data_ptr() if with_workspace else None,
+                                   ws_bytes if with_workspace else 0,
+                                   torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        torch.cuda.synchronize()
+        outs.append(y)
+    assert torch.equal(outs[0], outs[1])
+    _assert_within_one_ulp(outs[0], _exact(x, w, b, "tanh"))
     (y,) = ops.proj_grouped([(x, w, b, "tanh")])
-    _assert_within_one_ulp(y, _exact(x, w, b, "tanh"))
+    if with_workspace:
+        assert torch.equal(y, outs[0])
+
+
+@pytest.mark.parametrize("M,grows", [(1, False), (16, False), (17, True)])
+def test_workspace_only_where_it_is_used(dev, M, grows):
+    """proj_grouped allocates a split-k workspace above 16 rows alone."""
+    gen = torch.Generator().manual_seed(73)
+    x, w = _rand((M, 2048), gen, dev), _rand((1024, 2048), gen, dev, 1 / math.sqrt(2048))
+    y = torch.empty((M, 1024), dtype=torch.bfloat16, device=dev)
+    count = lambda: torch.cuda.memory_stats(dev)["allocation.all.allocated"]  # noqa: E731
+    before = count()
+    ops.proj_grouped([(x, w)], outs=[y])
+    assert (count() > before) == grows
+    _assert_within_one_ulp(y, _exact(x, w, None, None))

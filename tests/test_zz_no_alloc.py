@@ -3,9 +3,9 @@ nothing, its split-k partials in the library's static per-GPU buffer.
 
 Checked through the C ABI against wkv7_proj_grouped given the workspace it
 asks for (same plan, so the outputs must be bit-identical) and against the
-float64 product (within one bf16 ulp), on two calls in a row whose second
-input is smaller, both of which split k. The second call reuses the buffer the
-first one left its partials in."""
+float64 product (within one bf16 ulp), on calls in a row: two of few rows,
+which need no partials, and two that split k, the second one smaller, so that it
+reuses the buffer the first one left its partials in."""
 
 import math
 
@@ -69,6 +69,9 @@ def test_noalloc_matches_the_workspace_entry_point_on_two_calls(dev):
         (4, 2048, [2048, 96], [_lib.WKV7_ACT_NONE, _lib.WKV7_ACT_TANH]),
         # second call, smaller: one row, k = 1024, n = 1024
         (1, 1024, [1024], [_lib.WKV7_ACT_SIGMOID]),
+        # (both in the kernel of one row tile) and 20 rows, which do split
+        (20, 2048, [1000, 96], [_lib.WKV7_ACT_TANH, _lib.WKV7_ACT_NONE]),
+        (17, 1024, [1000], [_lib.WKV7_ACT_SIGMOID]),
     ]
     for M, K, ns, acts in cases:
         prods = _case(gen, dev, M, K, ns, acts)
@@ -80,7 +83,7 @@ def test_noalloc_matches_the_workspace_entry_point_on_two_calls(dev):
         arr = _groups([(x, w, b, y, a) for (x, w, b, a), y in zip(prods, ys)])
         ws_bytes = int(lib.wkv7_proj_workspace_bytes(M, ref_arr, len(prods)))
         assert 0 < ws_bytes <= _lib.WKV7_PROJ_STATIC_SCRATCH_BYTES, \
-            "the case must take the split-k path, within the static buffer"
+            "the case must ask for a split, within the static buffer"
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         assert lib.wkv7_proj_grouped(M, ref_arr, len(prods), ws.data_ptr(), ws_bytes,
                                      stream) == 0

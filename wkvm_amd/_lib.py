@@ -36,6 +36,7 @@ WKV7_TO_HOST = 0
 WKV7_FROM_HOST = 1
 WKV7_PROJ_MAX_GROUPS = 8
 WKV7_PROJ_STATIC_SCRATCH_BYTES = 8 * 1024 * 1024
+WKV7_PROJ_FEW_ROWS = 16
 WKV7_ACT_NONE = 0
 WKV7_ACT_TANH = 1
 WKV7_ACT_SIGMOID = 2

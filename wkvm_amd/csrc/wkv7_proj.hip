@@ -487,18 +487,19 @@ struct Plan {
 // against 9.4 in 32 x 32 tiles; o_proj of the 7B shape, 256, 12.2 against 13.5).
 // Its waves: 8 for long k, 4 where k has few chunks (LoRA up-projections of the
 // 7B shape 5.2 against 6.4 us).
-constexpr int kThinRows = 16, kThinShortK = 512;
+constexpr int kThinShortK = 512;
 
 int thin_waves(int64_t m, const wkv7_proj_group* gs, int ng, int cus) {
-  if (m > kThinRows) return 0;
+  if (m > WKV7_PROJ_FEW_ROWS) return 0;
   int kmax = 0;
   for (int i = 0; i < ng; ++i) kmax = std::max(kmax, gs[i].k);
   if (kmax <= kThinShortK) return 4;
   return count_tiles(m, gs, ng, kShapes[1]) * 2 <= int64_t(cus) ? 8 : 0;
 }
 
-// The plan of the tiled kernel (at 16 rows or fewer the thin one may run in its
-// place, and then leaves the workspace alone).
+// The plan of the tiled kernel. At 16 rows or fewer the thin one runs in its
+// place wherever it would split k (at most half a tile per unit of long k), so
+// the workspace is never used there.
 Plan make_plan(int64_t m, const wkv7_proj_group* gs, int ng, int cus) {
   int kmin = gs[0].k;
   int64_t cols = 0;

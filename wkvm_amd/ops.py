@@ -1250,7 +1250,8 @@ def proj_grouped(products: Sequence[tuple], outs: Sequence[torch.Tensor | None] 
     if M:
         lib = _lib.load()
         n = len(products)
-        ws_bytes = int(lib.wkv7_proj_workspace_bytes(M, groups, n))
+        ws_bytes = (int(lib.wkv7_proj_workspace_bytes(M, groups, n))
+                    if M > _lib.WKV7_PROJ_FEW_ROWS else 0)  # (never used up to there)
         ws = (torch.empty(ws_bytes, dtype=torch.uint8, device=ys[0].device) if ws_bytes
               else None)
         rc = lib.wkv7_proj_grouped(M, groups, n, _ptr(ws), ws_bytes,
