@@ -621,7 +621,6 @@ def bench_mixed(torch, dev, args, launcher):
     def step(order=lpt_t.data_ptr(), decode=True, concurrent=False):
         # concurrent: each layer's prefill on the main stream, then its decode
         # on a side stream forked from and joined into the main stream
-        # (WKV7Runner.mixed_step's schedule)
         if decode and concurrent:
             side.wait_stream(main)
         for l in range(L):

@@ -1,7 +1,7 @@
 """Config 4 against the oracle at its own workload: one scheduler step of the
 1.5B shape (H = 32) over a 1024-slot pool with 64 prefill rows of seeded
-lengths U[1, 2048] and 448 decode rows, through WKV7Runner.mixed_step with
-the decode launches on a side stream (the schedule bench.py times).
+lengths U[1, 2048] and 448 decode rows, through WKV7Runner.mixed_step (one
+prefill and one decode launch over the layers).
 
 The reference runs such a step as per-request prefill plus one batched decode
 (wkvm/engine.py:142-170) over ragged offsets (wkvm/core/mixed_batch.py:

@@ -440,9 +440,11 @@ def test_7b_shape_prefill_matches_oracle(dev, y_dtype):
     _check(pool.numpy(), ids, cu, U.vec_bits(vecs), gpool, y, zero_init=False)
 
 
-def test_mixed_step_concurrent_equals_serial(dev):
-    """The decode launches on a side stream (forked from and joined into the
-    current stream) give the same bits as the single-stream step."""
+@pytest.mark.parametrize("concurrent", [True, False])
+def test_mixed_step_equals_separate_launches(dev, concurrent):
+    """mixed_step's one decode and one prefill launch over all layers give the
+    bits of a decode and a prefill launch per layer; its `concurrent` argument
+    is accepted and changes nothing."""
     lay = RWKV7StateLayout(n_layer=3, hidden_size=512, num_heads=8, head_dim=64, head_v_dim=64,
                            dtype=torch.bfloat16)
     gen = synthetic.make_generator(62)
@@ -450,33 +452,31 @@ def test_mixed_step_concurrent_equals_serial(dev):
     init = synthetic.initial_states((3, S + 1, 8, 64, 64), gen).to(dev)
     dec_slots = list(range(2, 34, 2))
     pre_slots = [1, 5, 39]
-    lens = [700, 33, 1]
+    lens, cu = [700, 33, 1], [0, 700, 733, 734]
     dec_in = [synthetic.order(synthetic.wkv7_vectors((16, 8, 64), gen, device=dev))
               for _ in range(3)]
     pre_in = [synthetic.order(synthetic.wkv7_vectors((sum(lens), 8, 64), gen, device=dev))
               for _ in range(3)]
-    out = []
-    for concurrent in (True, False):
-        bank = RWKV7StateBank(lay, num_slots=S, device=dev)
-        bank.wkv.copy_(init)
-        ys = WKV7Runner(bank).mixed_step([{"wkv": s, "shift": s} for s in dec_slots], dec_in,
-                                         [{"wkv": s, "shift": s} for s in pre_slots], lens, pre_in,
-                                         concurrent=concurrent)
+    bank = RWKV7StateBank(lay, num_slots=S, device=dev)
+    bank.wkv.copy_(init)
+    dys, pys = WKV7Runner(bank).mixed_step([{"wkv": s, "shift": s} for s in dec_slots], dec_in,
+                                           [{"wkv": s, "shift": s} for s in pre_slots], lens,
+                                           pre_in, concurrent=concurrent)
+    for layer in range(3):
+        py = ops.wkv7_prefill_varlen(init[layer], pre_slots, cu, *pre_in[layer])
+        dy = ops.wkv7_decode_slots(init[layer], dec_slots, *dec_in[layer])
         torch.cuda.synchronize()
-        out.append((bank.wkv.clone(), ys))
-    assert torch.equal(out[0][0], out[1][0])
-    for a, b in zip(out[0][1][0] + out[0][1][1], out[1][1][0] + out[1][1][1]):
-        assert torch.equal(a, b)
+        assert torch.equal(pys[layer], py) and torch.equal(dys[layer], dy)
+    assert torch.equal(bank.wkv, init)
 
 
 @pytest.mark.parametrize("H", [64, 8])
-def test_large_batch_uses_the_64bit_input_path(dev, H):
-    """A batch whose input bytes exceed 31-bit offsets runs the operand waves'
-    global-load path instead of the buffer-resource one; the first (checked)
-    sequence must match the oracle there too. The second sequence is zero
-    input and only makes the batch large: 262,144 tokens at H = 64 (one
-    workgroup per head) or 2,097,152 at H = 8 (few heads: the quarter-head
-    kernel)."""
+def test_batch_of_more_than_31_bit_offsets(dev, H):
+    """A batch whose input bytes exceed 31-bit offsets: the row loads of its
+    long sequence move their base forward, and the first (checked) sequence
+    must match the oracle there too. The second sequence is zero input and only
+    makes the batch large: 262,144 tokens at H = 64 (half heads) or 2,097,152 at
+    H = 8 (quarter heads)."""
     S = 4
     lens = [300, (1 << 24) // H]
     cu = [0, lens[0], lens[0] + lens[1]]
@@ -607,6 +607,38 @@ def test_segmented_prefill_matches_oracle_and_one_pass(dev, zero_init, y_dtype):
     assert U.rel_l2(U.f64(gpool), U.f64(one)) <= 1e-4
     if y_dtype == torch.float32:
         assert U.rel_l2(U.f64(y), U.f64(y1)) <= 1e-4
+
+
+@pytest.mark.parametrize("segments", [5, 6, 7, 8])
+def test_more_than_four_segments_match_oracle(dev, segments):
+    """Five to eight segments per sequence (the counts that auto_segments takes
+    for few heads), of whole and of ragged length, from a non-zero state."""
+    H, lens = 2, [1000, 16 * segments, 90]
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    gen = synthetic.make_generator(63)
+    pool = synthetic.initial_states((4, H, 64, 64), gen)
+    ids = [3, 0, 2]
+    vecs = synthetic.wkv7_vectors((int(cu[-1]), H, 64), gen)
+    gpool = pool.to(dev)
+    y = ops.wkv7_prefill_segments(gpool, ids, cu.tolist(), *(vecs[n].to(dev) for n in "rwkvab"),
+                                  segments=segments, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    _check(pool.numpy(), ids, cu, U.vec_bits(vecs), gpool, y, False)
+    assert torch.equal(gpool[1].cpu(), pool[1])
+
+
+def test_fla_signature_takes_eight_segments(dev):
+    """One sequence of few heads and 1,024 tokens per segment through the
+    fla signature, against the oracle."""
+    T, H = 8192, 1
+    assert ops.auto_segments(H, [T], dev) == 8 and ops.auto_segments(H, [T // 2], dev) == 4
+    gen = synthetic.make_generator(65)
+    vecs = synthetic.wkv7_vectors((1, T, H, 64), gen)
+    o, hT = ops.chunk_rwkv7(*[vecs[n].to(dev) for n in "rwkvab"])
+    y_ref, h_ref = O.scan_bf16(np.array([0, T]), *[U.bits(vecs[n][0]) for n in "rwkvab"],
+                               pool=None, slot_ids=None)
+    assert U.rel_l2(U.f64(hT), h_ref) <= REL_L2
+    assert U.rel_l2(U.f64(o[0]), O.round_f64_to_bf16(y_ref)) <= REL_L2
 
 
 def test_runner_segmented_prefill_matches_one_pass(dev):
@@ -994,3 +1026,29 @@ def test_segmented_prefill_keeps_value_columns_apart(dev):
     assert torch.equal(got[0][0][..., rest], got[1][0][..., rest])
     assert torch.equal(got[0][1][..., rest], got[1][1][..., rest])
     assert got[1][0][..., col].isnan().all()
+
+
+def test_state_split_over_the_whole_range(dev):
+    """The state enters its products as bf16 hi + lo, lo from x - hi by a
+    two-element dot product. Read out with a one-hot r, y (fp32) is hi + lo:
+    exactly that for x of every exponent from 2^-100 up to bf16's largest and of
+    random mantissas and signs, next to neighbours of any other exponent."""
+    H, n = 8, 16
+    g = torch.Generator().manual_seed(93)
+    shape = (n, H, 64, 64)
+    bits = (torch.randint(0, 1 << 23, shape, generator=g)
+            | torch.randint(127 - 100, 254, shape, generator=g) << 23)
+    x = bits.int().view(torch.float32) * (torch.randint(0, 2, shape, generator=g) * 2 - 1)
+    T = 64
+    r = torch.eye(64).repeat(n, 1).view(n * T, 1, 64).expand(-1, H, -1).contiguous()
+    zero = torch.zeros_like(r, dtype=torch.bfloat16)
+    xs = [t.to(dev) for t in (r.bfloat16(), zero, zero, zero, zero, zero)]
+    pool = x.to(dev)
+    y = ops.wkv7_prefill_varlen(pool, list(range(n)), [T * i for i in range(n + 1)], *xs,
+                                out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    assert torch.equal(pool.cpu(), x)
+    hi = x.bfloat16().float()
+    want = hi + (x - hi).bfloat16().float()
+    got = y.cpu().view(n, T, H, 64).transpose(1, 2)
+    assert torch.equal(got, want)

@@ -38,9 +38,11 @@ __device__ __forceinline__ uint2 ld_tr(const uint16_t* p) {
 
 // x = hi + lo: hi = bf16(x) and lo = bf16(x - hi), both rounded to nearest
 // even; |x - hi - lo| <= 2^-18 |x|. The difference comes from one
-// v_dot2_f32_bf16 with {-1, 0} or {0, -1}, exact in fp32 (checked against the
-// subtraction over the whole range on gfx950, denormals included) and one
-// instruction where unpacking hi and subtracting take two. The constants
+// v_dot2_f32_bf16 with {-1, 0} or {0, -1}, one instruction where unpacking hi
+// and subtracting take two. It is exact in fp32 (x - hi has at most 16
+// significant bits), except that the pair's other half enters times 0: one that
+// is not finite makes the difference NaN, so the two values of a pair belong
+// to one value column of the state, or to one token. The constants
 // must be registers: as literals the compiler encodes {-1, 0} as the inline
 // constant -1.0, which the instruction reads as {0, -1}.
 struct Neg {

@@ -32,6 +32,12 @@ LayerInputs = Sequence[torch.Tensor]  # (r, w, k, v, a, b)
 
 
 class WKV7Runner:
+    """The WKV7 work of whole requests over a bank, every layer at once: each
+    call takes all layers' vectors and launches one kernel over them. (A model
+    whose next layer needs this one's output has one layer's vectors at a time;
+    it calls the bank's ``decode_wkv`` / ``prefill_wkv`` per layer, or keeps
+    whole time-mix blocks in a ``TimeMixDecodeGraph``.)"""
+
     # Chunks at least this long run segmented when ``prefill_segments`` is a
     # count (one layer's segments are faster from about 2k tokens on).
     SEGMENT_MIN_TOKENS = 2048
@@ -140,11 +146,12 @@ class WKV7Runner:
         Returns ``(decode_ys, prefill_ys)`` per layer.
 
         One prefill launch and one decode launch over all layers, both on the
-        caller's stream whether ``concurrent`` or not: with one launch per
-        kind there is one ragged tail to fill instead of one per layer, and
-        decode workgroups on a second stream take units from the prefill's
-        next workgroups (two layers of 64 prompts and 448 decode rows, 1.5B
-        shape: 1175 us on one stream, 1220 us on two)."""
+        caller's stream: with one launch per kind there is one ragged tail to
+        fill instead of one per layer, and decode workgroups on a second stream
+        take units from the prefill's next workgroups (two layers of 64 prompts
+        and 448 decode rows, 1.5B shape: 1175 us on one stream, 1220 us on two).
+        ``concurrent``, which asked for that second stream, is still accepted
+        and has no effect."""
         self._check_layers(decode_inputs)
         self._check_layers(prefill_inputs)
         if len(prefill_lens) != len(prefill_batch):
