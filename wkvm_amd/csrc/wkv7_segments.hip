@@ -132,8 +132,9 @@ __global__ __launch_bounds__(kCombThreads) void segment_correct_kernel(
           acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(
               hs[(32 * kb + 8 * lg + e) * kHinPitch + 16 * ct + li], qv[kb][e >> 2][e & 3],
               acc[ct], 0, 0, 0);
-    // past the last product's 8 passes before a vector instruction reads it
-    asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+    // past the last product's 8 passes before a vector instruction reads it (the
+    // accumulators as "a": with "v" they would be read back ahead of the wait)
+    asm volatile("s_nop 15" : "+a"(acc[0]), "+a"(acc[1]), "+a"(acc[2]), "+a"(acc[3]));
   }
   if (!mine) return;
 #pragma unroll
