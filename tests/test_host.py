@@ -261,6 +261,52 @@ def test_fla_op_holds_its_plan_across_the_launch(monkeypatch):
     assert held == [True]
 
 
+def test_replay_order_waits_only_across_streams(monkeypatch):
+    """One stream: no event, no wait. Another one: the device once, then each
+    call behind the one before it. Under capture the replay alone."""
+    log, now = [], {}
+
+    class Stream:
+        def __init__(self, name):
+            self.name = name
+
+        def wait_event(self, event):
+            log.append((self.name, "waits for", event.at))
+
+    class Event:
+        at = None
+
+        def record(self, stream):
+            self.at = stream.name
+            log.append((stream.name, "records"))
+
+    class Graph:
+        @staticmethod
+        def replay():
+            log.append((now["s"].name, "replays"))
+
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev: now["s"])
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda dev: log.append("device"))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: now["capturing"])
+    monkeypatch.setattr(ops, "_stream_ptr", lambda dev: id(now["s"]))
+    order, a, b = ops.ReplayOrder(), Stream("a"), Stream("b")
+
+    def replay(stream, capturing=False):
+        now.update(s=stream, capturing=capturing)
+        log.clear()
+        order.replay(Graph(), torch.device("cpu"))
+        return list(log)
+
+    assert replay(a) == replay(a) == [("a", "replays")]
+    assert replay(b, capturing=True) == [("b", "replays")]
+    assert replay(a) == [("a", "replays")]
+    assert replay(b) == ["device", ("b", "waits for", None), ("b", "replays"), ("b", "records")]
+    assert replay(a) == [("a", "waits for", "b"), ("a", "replays"), ("a", "records")]
+    assert replay(a) == [("a", "waits for", "a"), ("a", "replays"), ("a", "records")]
+    assert replay(b, capturing=True) == [("b", "replays")]
+
+
 def test_longest_first_order():
     # lengths 3, 0, 9, 3, 5: longest first, equal lengths in index order
     assert ops.longest_first([0, 3, 3, 12, 15, 20]) == [2, 4, 0, 3, 1]

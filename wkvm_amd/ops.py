@@ -140,6 +140,8 @@ class ReplayOrder:
         self._leave(stream)
 
     def replay(self, graph: torch.cuda.CUDAGraph, device: torch.device) -> None:
+        if torch.cuda.is_current_stream_capturing():
+            return graph.replay()  # runs when its own graph does: nothing to order yet
         stream = self._enter(device)
         graph.replay()
         self._leave(stream)
